@@ -135,6 +135,23 @@ int w8a8_quant_rows(const void* x, int x_dtype, int64_t rows, int64_t k, int64_t
                     int8_t* q, int64_t ldq, float* scales, hipStream_t stream);
 
 /*
+ * Quantize-dequantize in one pass, one dynamic scale per row and group of
+ * `group` columns (0, or at least k: the whole row; the last group may be
+ * shorter):
+ *   scales[r, g] = scale_from_absmax(max over the group |x[r, k]|)
+ *   q[r, k]      = quantize_symmetric(x[r, k], scales[r, g])   (q nullable)
+ *   deq[r, k]    = x_dtype(f32(q[r, k]) * scales[r, g])
+ * Replaces dynamic_per_token_activation_qdq (w8a8.py:106-115),
+ * per_output_weight_qdq (w8a8.py:53-62) and groupwise_weight_qdq
+ * (w8a8.py:65-91) with their dequantized results.
+ * x: [rows, ldx], deq: [rows, ld_deq], both of x_dtype (F32/F16/BF16); q: int8
+ * [rows, ldq]; scales: [rows, ceil(k / group)].
+ */
+int w8a8_qdq_rows(const void* x, int x_dtype, int64_t rows, int64_t k, int64_t ldx,
+                  int64_t group, int8_t* q, int64_t ldq, void* deq, int64_t ld_deq,
+                  float* scales, hipStream_t stream);
+
+/*
  * quantize_symmetric (w8a8.py:33-43) with caller scales: scale[r * scale_stride]
  * (scale_stride 0: one per-tensor scale, the static_activation_qdq case,
  * w8a8.py:101-103).  Scales must be positive; the caller checks that, as the

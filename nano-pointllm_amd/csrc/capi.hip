@@ -497,6 +497,20 @@ int w8a8_quant_rows(const void* x, int x_dtype, int64_t rows, int64_t k, int64_t
                                      scales, stream));
 }
 
+int w8a8_qdq_rows(const void* x, int x_dtype, int64_t rows, int64_t k, int64_t ldx, int64_t group,
+                  int8_t* q, int64_t ldq, void* deq, int64_t ld_deq, float* scales,
+                  hipStream_t stream) {
+  if (rows < 0 || k < 0 || rows > kMaxRows || k > kMaxRows || group < 0) return W8A8_ERR_SHAPE;
+  if (!float_dtype(x_dtype)) return W8A8_ERR_DTYPE;
+  if (rows == 0 || k == 0) return W8A8_OK;
+  if (x == nullptr || deq == nullptr || scales == nullptr) return W8A8_ERR_NULL;
+  if (ldx < k || ld_deq < k || (q != nullptr && ldq < k)) return W8A8_ERR_SHAPE;
+  const uintptr_t es = static_cast<uintptr_t>(elem_size(x_dtype));
+  if (!aligned(x, es) || !aligned(deq, es) || !aligned(scales, 4)) return W8A8_ERR_ALIGN;
+  return status_of(launch_qdq_rows(x, x_dtype, ldx, rows, k, group == 0 || group > k ? k : group, q,
+                                   ldq, deq, ld_deq, scales, stream));
+}
+
 int w8a8_quant_rows_scaled(const void* x, int x_dtype, int64_t rows, int64_t k, int64_t ldx,
                            const float* scale, int64_t scale_stride, int8_t* q, int64_t ldq,
                            hipStream_t stream) {

@@ -9,6 +9,8 @@
 // row of a row-major matrix".
 #include "w8a8_internal.h"
 
+#include <type_traits>
+
 namespace w8a8 {
 
 namespace {
@@ -253,6 +255,185 @@ __global__ __launch_bounds__(NT) void quant_rows_parts_kernel(
   }
 }
 
+// |x|max over the LPG lanes of a power-of-two group (every lane active; all
+// its lanes end with the result).  Within a row of 16 the partners come from
+// DPP quad permutations and mirrors (a mirror pairs each lane with one of the
+// other half, which holds that half's maximum after the levels below), past
+// it from the permlane swaps of wave_butterfly.
+template <int LPG>
+__device__ inline float group_max_abs(float v) {
+  constexpr int kQuadXor1 = 0xb1, kQuadXor2 = 0x4e, kRowHalfMirror = 0x141, kRowMirror = 0x140;
+  auto dpp = [&](auto ctrl) {
+    const uint32_t u = __builtin_amdgcn_update_dpp(0u, __float_as_uint(v), decltype(ctrl)::value,
+                                                   0xf, 0xf, false);
+    v = fmaxf(v, __uint_as_float(u));
+  };
+  if constexpr (LPG >= 2) dpp(std::integral_constant<int, kQuadXor1>{});
+  if constexpr (LPG >= 4) dpp(std::integral_constant<int, kQuadXor2>{});
+  if constexpr (LPG >= 8) dpp(std::integral_constant<int, kRowHalfMirror>{});
+  if constexpr (LPG >= 16) dpp(std::integral_constant<int, kRowMirror>{});
+  if constexpr (LPG >= 32) {
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  }
+  if constexpr (LPG >= 64) {
+    const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  }
+  return v;
+}
+
+// Quantize-dequantize outputs of one 8-column chunk: int8 values (q nullable)
+// and q * s rounded to the input type, the columns below K.
+struct QdqOut {
+  int8_t* q;
+  int64_t ldq;
+  void* deq;
+  int64_t ldd;
+  int vec_q, vec_d;
+};
+
+template <typename TX>
+__device__ inline void qdq_store8(const QdqOut& o, int64_t row, int64_t k0, int valid,
+                                  const float (&v)[8], float s, float r) {
+  int32_t qi[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) qi[j] = quant_elem<TX>(v[j], s, r, true);
+  if (o.q != nullptr) {
+    int8_t* dst = o.q + row * o.ldq + k0;
+    if (o.vec_q && valid >= 8) {
+      *reinterpret_cast<u32x2*>(dst) =
+          u32x2{pack4_i8(qi[0], qi[1], qi[2], qi[3]), pack4_i8(qi[4], qi[5], qi[6], qi[7])};
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        if (j < valid) dst[j] = static_cast<int8_t>(qi[j]);
+    }
+  }
+  float d[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) d[j] = __fmul_rn(static_cast<float>(qi[j]), s);
+  TX* dst = static_cast<TX*>(o.deq) + row * o.ldd + k0;
+  if (o.vec_d && valid >= 8) {
+    if constexpr (sizeof(TX) == 2) {
+      *reinterpret_cast<u32x4*>(dst) = u32x4{pack2_bits<TX>(d[0], d[1]), pack2_bits<TX>(d[2], d[3]),
+                                             pack2_bits<TX>(d[4], d[5]), pack2_bits<TX>(d[6], d[7])};
+    } else {
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        reinterpret_cast<u32x4*>(dst)[h] =
+            u32x4{__float_as_uint(d[4 * h]), __float_as_uint(d[4 * h + 1]),
+                  __float_as_uint(d[4 * h + 2]), __float_as_uint(d[4 * h + 3])};
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      if (j < valid) dst[j] = from_f32<TX>(d[j]);
+  }
+}
+
+// Quantize-dequantize with one scale per row and group of 8 LPG columns
+// (groupwise_weight_qdq, w8a8.py:65-91): LPG adjacent lanes hold a group, one
+// 8-column chunk each, so a group's scale takes log2(LPG) lane exchanges and
+// the matrix is read and written once.  Bound: HBM (2 bytes in, 3 out per
+// 16-bit weight): 4096 x 11008 bfloat16 in groups of 128 takes 44.5 us, 5.1
+// TB/s, a large copy's rate on this card; a workgroup per group (quantization
+// alone 230 us) and torch's elementwise passes behind it took 602.
+template <typename TX, int LPG>
+__global__ __launch_bounds__(kQuantThreads) void qdq_groups_kernel(
+    const TX* __restrict__ x, int64_t ldx, int64_t K, int vec_in, int groups, int blocks_per_row,
+    QdqOut out, float* __restrict__ scales_out) {
+  const int64_t row = blockIdx.x / blocks_per_row;
+  const int chunk =
+      static_cast<int>(blockIdx.x % blocks_per_row) * kQuantThreads + static_cast<int>(threadIdx.x);
+  const int64_t k0 = static_cast<int64_t>(chunk) * 8;
+  const int valid = static_cast<int>(K - k0 <= 0 ? 0 : (K - k0 < 8 ? K - k0 : 8));
+  float v[8];
+  load8(x + row * ldx + k0, v, vec_in != 0, valid);
+  float amax = 0.0f;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(v[j]));
+  amax = group_max_abs<LPG>(amax);
+  const float s = scale_from_absmax(amax);
+  const float r = 1.0f / s;
+  if (valid > 0) {
+    if (chunk % LPG == 0) scales_out[row * groups + chunk / LPG] = s;
+    qdq_store8<TX>(out, row, k0, valid, v, s, r);
+  }
+}
+
+// Quantize-dequantize with one workgroup per (row, group): whole rows
+// (dynamic_per_token_activation_qdq, per_output_weight_qdq) and the group
+// sizes the kernel above does not take.  The group stays in REG chunks per
+// thread between the absmax and the outputs (REG 0: it is read twice).
+// Latency-bound at activation sizes: 560 x 4096 bfloat16 as a call takes 15.2
+// us, mostly the host's, against 31.2 for quant_rows_kernel (4.8 us) and three
+// elementwise passes (20 us).
+template <typename TX, int REG, int NT>
+__global__ __launch_bounds__(NT) void qdq_rows_kernel(const TX* __restrict__ x, int64_t ldx,
+                                                      int64_t K, int64_t group, int vec_in,
+                                                      int groups, QdqOut out,
+                                                      float* __restrict__ scales_out) {
+  __shared__ float red[NT / 64];
+  const int64_t row = blockIdx.x / groups;
+  const int64_t c0 = static_cast<int64_t>(blockIdx.x % groups) * group;
+  const int64_t n = K - c0 < group ? K - c0 : group;  // columns of this group
+  const int tid = threadIdx.x;
+  const TX* xr = x + row * ldx + c0;
+  out.q = out.q != nullptr ? out.q + c0 : nullptr;
+  out.deq = static_cast<TX*>(out.deq) + c0;
+  const int64_t nchunk = (n + 7) / 8;
+  auto valid_of = [&](int64_t k0) { return static_cast<int>(n - k0 <= 0 ? 0 : (n - k0 < 8 ? n - k0 : 8)); };
+  float v[REG > 0 ? REG : 1][8];
+  float amax = 0.0f;
+  if constexpr (REG > 0) {
+    if (vec_in) {
+      load_row_chunks<TX, REG, NT>(xr, n, tid, v);
+    } else {
+#pragma unroll
+      for (int c = 0; c < REG; ++c) {
+        const int64_t k0 = (tid + static_cast<int64_t>(c) * NT) * 8;
+        load8(xr + k0, v[c], false, valid_of(k0));
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < REG; ++c)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(v[c][j]));
+  } else {
+    for (int64_t c = tid; c < nchunk; c += NT) {
+      load8(xr + c * 8, v[0], vec_in != 0, valid_of(c * 8));
+#pragma unroll
+      for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(v[0][j]));
+    }
+  }
+  amax = wave_max_abs(amax);
+  if constexpr (NT > 64) {
+    if ((tid & 63) == 0) red[tid >> 6] = amax;
+    __syncthreads();
+    amax = red[0];
+#pragma unroll
+    for (int w = 1; w < NT / 64; ++w) amax = fmaxf(amax, red[w]);
+  }
+  const float s = scale_from_absmax(amax);
+  const float r = 1.0f / s;
+  if (tid == 0) scales_out[blockIdx.x] = s;
+  if constexpr (REG > 0) {
+#pragma unroll
+    for (int c = 0; c < REG; ++c) {
+      const int64_t k0 = (tid + static_cast<int64_t>(c) * NT) * 8;
+      const int valid = valid_of(k0);
+      if (valid > 0) qdq_store8<TX>(out, row, k0, valid, v[c], s, r);
+    }
+  } else {
+    for (int64_t c = tid; c < nchunk; c += NT) {
+      const int valid = valid_of(c * 8);
+      load8(xr + c * 8, v[0], vec_in != 0, valid);
+      qdq_store8<TX>(out, row, c * 8, valid, v[0], s, r);
+    }
+  }
+}
+
 // Packs a row-major int8 [rows, K] matrix into 16x64 tiles.  One thread per
 // 16-byte lane slot.  layout 1 maps packed row p to source row p/2 (p even)
 // or rows/2 + p/2 (p odd): the gate/up "interleave" order of
@@ -429,6 +610,72 @@ hipError_t launch_quant_rows(const void* x, int x_dtype, int64_t ldx, int64_t ro
 }
 
 template <typename TX, int NT>
+void qdq_rows_launch(dim3 g, hipStream_t st, const TX* x, int64_t ldx, int64_t K, int64_t group,
+                     int vec_in, int groups, const QdqOut& out, float* scales) {
+  const int64_t per = ceil_div(group < K ? group : K, 8 * NT);
+#define W8A8_QDQ_REG(R)                                                                          \
+  hipLaunchKernelGGL((qdq_rows_kernel<TX, R, NT>), g, dim3(NT), 0, st, x, ldx, K, group, vec_in, \
+                     groups, out, scales)
+  if (per <= 1)
+    W8A8_QDQ_REG(1);
+  else if (per <= 2)
+    W8A8_QDQ_REG(2);
+  else if (per <= 4)
+    W8A8_QDQ_REG(4);
+  else if (per <= kRegChunksMax)
+    W8A8_QDQ_REG(kRegChunksMax);
+  else
+    W8A8_QDQ_REG(0);
+#undef W8A8_QDQ_REG
+}
+
+// Groups of 8, 16, .. 512 columns run on qdq_groups_kernel; other groups take
+// a workgroup each: one wavefront up to 512 columns, 256 threads past that.
+template <typename TX>
+hipError_t qdq_dispatch(const TX* x, int64_t ldx, int64_t rows, int64_t K, int64_t group,
+                        const QdqOut& o, float* scales, hipStream_t st) {
+  const int64_t groups = ceil_div(K, group);
+  QdqOut out = o;
+  const bool cols8 = K % 8 == 0 && group % 8 == 0;
+  const int vec_in = cols8 && aligned16(x) && ldx % 8 == 0;
+  out.vec_q = cols8 && aligned8(o.q) && o.ldq % 8 == 0;
+  out.vec_d = cols8 && aligned16(o.deq) && o.ldd % 8 == 0;
+  const int64_t lanes = group / 8;
+  if (group % 8 == 0 && lanes <= 64 && (lanes & (lanes - 1)) == 0 && groups > 1) {
+    const int64_t bpr = ceil_div(groups * lanes, kQuantThreads);
+    if (rows * bpr > INT32_MAX) return hipErrorInvalidConfiguration;
+#define W8A8_QDQ_LPG(L)                                                                        \
+  case L:                                                                                      \
+    hipLaunchKernelGGL((qdq_groups_kernel<TX, L>), dim3(static_cast<unsigned>(rows * bpr)),    \
+                       dim3(kQuantThreads), 0, st, x, ldx, K, vec_in, static_cast<int>(groups), \
+                       static_cast<int>(bpr), out, scales);                                    \
+    break
+    switch (lanes) {
+      W8A8_QDQ_LPG(1);
+      W8A8_QDQ_LPG(2);
+      W8A8_QDQ_LPG(4);
+      W8A8_QDQ_LPG(8);
+      W8A8_QDQ_LPG(16);
+      W8A8_QDQ_LPG(32);
+      W8A8_QDQ_LPG(64);
+    }
+#undef W8A8_QDQ_LPG
+    return hipGetLastError();
+  }
+  if (rows * groups > INT32_MAX) return hipErrorInvalidConfiguration;
+  const dim3 g(static_cast<unsigned>(rows * groups));
+  const int64_t n = group < K ? group : K;
+  const int ng = static_cast<int>(groups);
+  if (n <= 512)
+    qdq_rows_launch<TX, 64>(g, st, x, ldx, K, group, vec_in, ng, out, scales);
+  else if (rows * groups <= 2048 && n > 8 * kQuantThreads)
+    qdq_rows_launch<TX, 2 * kQuantThreads>(g, st, x, ldx, K, group, vec_in, ng, out, scales);
+  else
+    qdq_rows_launch<TX, kQuantThreads>(g, st, x, ldx, K, group, vec_in, ng, out, scales);
+  return hipGetLastError();
+}
+
+template <typename TX, int NT>
 void quant_parts_launch(dim3 g, hipStream_t st, int64_t chunks, const TX* x, int64_t ldx,
                         int64_t K, int vec_in, const float* parts, int64_t nparts, int8_t* q,
                         int64_t ldq, int vec_out, float* scales) {
@@ -484,6 +731,24 @@ hipError_t launch_quant_rows_parts(const void* x, int x_dtype, int64_t ldx, int6
     case kBF16:
       return quant_parts_dispatch(static_cast<const __hip_bfloat16*>(x), ldx, rows, K, parts,
                                   nparts, q, ldq, scales_out, st);
+    default:
+      return hipErrorInvalidValue;
+  }
+}
+
+hipError_t launch_qdq_rows(const void* x, int x_dtype, int64_t ldx, int64_t rows, int64_t K,
+                           int64_t group, int8_t* q, int64_t ldq, void* deq, int64_t ldd,
+                           float* scales_out, hipStream_t st) {
+  if (rows == 0 || K == 0) return hipSuccess;
+  const QdqOut out{q, ldq, deq, ldd, 0, 0};
+  switch (x_dtype) {
+    case kF32:
+      return qdq_dispatch(static_cast<const float*>(x), ldx, rows, K, group, out, scales_out, st);
+    case kF16:
+      return qdq_dispatch(static_cast<const __half*>(x), ldx, rows, K, group, out, scales_out, st);
+    case kBF16:
+      return qdq_dispatch(static_cast<const __hip_bfloat16*>(x), ldx, rows, K, group, out,
+                          scales_out, st);
     default:
       return hipErrorInvalidValue;
   }

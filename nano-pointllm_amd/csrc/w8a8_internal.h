@@ -106,6 +106,14 @@ hipError_t launch_quant_rows_parts(const void* x, int x_dtype, int64_t ldx, int6
                                    int64_t K, const float* parts, int64_t nparts, int8_t* q,
                                    int64_t ldq, float* scales_out, hipStream_t st);
 
+// Quantize-dequantize in one pass: per row and group of `group` columns (the
+// last may be shorter) a dynamic scale, int8 values (q nullable, [rows, ldq])
+// and q * scale rounded to x's type (deq [rows, ldd]); scales_out
+// [rows, ceil(K / group)].
+hipError_t launch_qdq_rows(const void* x, int x_dtype, int64_t ldx, int64_t rows, int64_t K,
+                           int64_t group, int8_t* q, int64_t ldq, void* deq, int64_t ldd,
+                           float* scales_out, hipStream_t st);
+
 hipError_t launch_pack_rows(const int8_t* src, int64_t rows, int64_t K, int64_t ld, int layout,
                             int8_t* dst, hipStream_t st);
 

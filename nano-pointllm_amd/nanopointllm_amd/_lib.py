@@ -46,6 +46,7 @@ EXPORTED_SYMBOLS = (
     "w8a8_workspace_bytes",
     "w8a8_gemm_tile_config",
     "w8a8_quant_rows",
+    "w8a8_qdq_rows",
     "w8a8_quant_rows_scaled",
     "w8a8_pack_rows",
     "w8a8_gemm_i32",
@@ -82,6 +83,7 @@ _SIGNATURES = {
     "w8a8_workspace_bytes": (_i64, [_i64, _i64]),
     "w8a8_gemm_tile_config": (_int, [_i64, _i64, _i64]),
     "w8a8_quant_rows": (_int, [_vp, _int, _i64, _i64, _i64, _vp, _i64, _vp, _vp]),
+    "w8a8_qdq_rows": (_int, [_vp, _int, _i64, _i64, _i64, _i64, _vp, _i64, _vp, _i64, _vp, _vp]),
     "w8a8_quant_rows_scaled": (_int, [_vp, _int, _i64, _i64, _i64, _vp, _i64, _vp, _i64, _vp]),
     "w8a8_pack_rows": (_int, [_vp, _i64, _i64, _i64, _int, _vp, _vp]),
     "w8a8_gemm_i32": (_int, [_vp, _i64, _vp, _vp, _i64, _i64, _i64, _i64, _vp, _i64, _vp]),

@@ -3,8 +3,8 @@
 Mirrors the function API of ``nanopointllm.compression.w8a8``
 (nanopointllm/compression/w8a8.py) for CUDA tensors: same names, same
 argument meaning, same results, same error messages.  Every integer result is
-produced by the HIP kernels; torch is used only for device memory, reshapes
-and the trivial elementwise QDQ reconstruction (``q * s``).
+produced by the HIP kernels, dynamic QDQ reconstructions too; torch is used only
+for device memory, reshapes and the static QDQ's elementwise ``q * s``.
 """
 from __future__ import annotations
 
@@ -78,6 +78,26 @@ def quant_rows(x: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
                                        q.data_ptr(), max(k, 1), s.data_ptr(),
                                        _lib.stream_handle(device)), "w8a8_quant_rows")
     return q.reshape(x.shape), s.reshape(x.shape[:-1])
+
+
+def qdq_rows(x: torch.Tensor, *, group_size: int | None = None, want_q: bool = True
+             ) -> tuple[torch.Tensor, torch.Tensor | None, torch.Tensor]:
+    """Dynamic quantize-dequantize of ``x[..., K]`` in one kernel, one scale per
+    row, or per row and ``group_size`` columns: ``(dequantized rows of x's
+    dtype, int8 rows or None, f32 scales [rows, groups])``, the rows 2-D."""
+    device = _lib.require_cuda(x)
+    x2, ldx = _rows_view(x)
+    rows, k = x2.shape
+    group = k if group_size is None else min(group_size, k)
+    groups = -(-k // group) if k else 0
+    deq = torch.empty((rows, k), dtype=x.dtype, device=device)
+    q = torch.empty((rows, k), dtype=torch.int8, device=device) if want_q else None
+    s = torch.empty((rows, groups), dtype=torch.float32, device=device)
+    if rows and k:
+        _lib.check(_lib.load().w8a8_qdq_rows(
+            x2.data_ptr(), _lib.dtype_code(x2.dtype), rows, k, ldx, group, _lib.ptr(q), k,
+            deq.data_ptr(), k, s.data_ptr(), _lib.stream_handle(device)), "w8a8_qdq_rows")
+    return deq, q, s
 
 
 def quant_rows_scaled(x: torch.Tensor, scale: torch.Tensor) -> torch.Tensor:
@@ -637,10 +657,9 @@ def dynamic_per_token_activation_qdq(values: torch.Tensor, *, axis: int = -1
     if values.dim() == 0:
         raise ValueError("dynamic per-token quantization expects a tensor")
     moved = values.movedim(axis, -1)
-    q, s = quant_rows(moved)
-    scales = s.unsqueeze(-1)
-    qdq = (q.float() * scales).to(values.dtype)
-    return qdq.movedim(-1, axis), scales.movedim(-1, axis)
+    qdq, _, s = qdq_rows(moved, want_q=False)
+    scales = s.reshape(*moved.shape[:-1], 1)
+    return qdq.reshape(moved.shape).movedim(-1, axis), scales.movedim(-1, axis)
 
 
 def per_output_weight_qdq(weight: torch.Tensor
@@ -649,42 +668,31 @@ def per_output_weight_qdq(weight: torch.Tensor
     if weight.dim() < 2:
         raise ValueError("weight must have at least two dimensions")
     rows = weight.detach().reshape(weight.shape[0], -1)
-    q, scales = quant_rows(rows)
-    deq = (q.float() * scales[:, None]).reshape_as(weight)
-    return deq.to(weight.dtype), q.reshape_as(weight), scales
+    deq, q, scales = qdq_rows(rows)
+    return deq.reshape_as(weight), q.reshape_as(weight), scales.reshape(-1)
 
 
 def groupwise_weight_qdq(weight: torch.Tensor, *, group_size: int = 128
                          ) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
     """``groupwise_weight_qdq`` (w8a8.py:65-91): one scale per row and group of
     ``group_size`` input columns (the last group may be shorter).  Returns
-    (dequant, int8, f32 scales [rows, groups]).  Each group is a strided
-    [rows, group] view quantized per row by the HIP kernel."""
+    (dequant, int8, f32 scales [rows, groups]), written by one kernel.  A
+    weight type that the kernels do not take goes through binary32."""
     if weight.dim() < 2:
         raise ValueError("groupwise W8 expects at least two weight dimensions")
     if group_size <= 0:
         raise ValueError("group_size must be positive")
-    device = _lib.require_cuda(weight)
-    rows = weight.shape[0]
-    flat = weight.detach().reshape(rows, -1)
-    cols = flat.shape[1]
-    groups = (cols + group_size - 1) // group_size
-    q = torch.empty((rows, cols), dtype=torch.int8, device=device)
-    deq = torch.empty((rows, cols), dtype=weight.dtype, device=device)
-    scales = torch.empty((rows, groups), dtype=torch.float32, device=device)
-    full = cols // group_size
-    if full:
-        body = flat[:, : full * group_size].float().reshape(rows * full, group_size)
-        qb, sb = quant_rows(body)
-        q[:, : full * group_size] = qb.reshape(rows, full * group_size)
-        scales[:, :full] = sb.reshape(rows, full)
-    if full < groups:
-        qt, st = quant_rows(flat[:, full * group_size:].float())
-        q[:, full * group_size:] = qt
-        scales[:, full] = st
-    per_col = scales.repeat_interleave(group_size, dim=1)[:, :cols]
-    deq.copy_((q.float() * per_col).to(weight.dtype))
-    return deq.reshape(weight.shape), q.reshape(weight.shape), scales
+    _lib.require_cuda(weight)
+    flat = weight.detach().reshape(weight.shape[0], -1)
+    if flat.dtype not in (torch.float32, torch.float16, torch.bfloat16):
+        flat = flat.float()
+    if flat.numel() == 0:
+        q = torch.empty(flat.shape, dtype=torch.int8, device=flat.device)
+        scales = torch.empty((flat.shape[0], -(-flat.shape[1] // group_size)),
+                             dtype=torch.float32, device=flat.device)
+        return torch.empty_like(weight), q.reshape(weight.shape), scales
+    deq, q, scales = qdq_rows(flat, group_size=group_size)
+    return deq.to(weight.dtype).reshape(weight.shape), q.reshape(weight.shape), scales
 
 
 def tensor_error(reference: torch.Tensor, candidate: torch.Tensor) -> dict[str, float]:
