@@ -175,6 +175,19 @@ int w8a8_pack_rows(const int8_t* src, int64_t rows, int64_t k, int64_t ld, int l
                    int8_t* packed, hipStream_t stream);
 
 /*
+ * w8a8_quant_rows and w8a8_pack_rows in one pass: the rows of n_src (1..3)
+ * row-major matrices x[i] [x_rows[i], ldx[i]] of x_dtype (F32/F16/BF16, k
+ * columns each) are quantized with a dynamic scale per row and written
+ * straight into the packed tiles, one matrix after another
+ * (W8A8_ROWS_AS_IS), or alternating rows of one [gate; up] matrix or of two
+ * of equal rows (W8A8_ROWS_INTERLEAVE_HALVES).  scales: [rows], in packed row
+ * order.  x, x_rows and ldx are host arrays, read before the call returns.
+ */
+int w8a8_quant_pack_rows(const void* const* x, const int64_t* x_rows, const int64_t* ldx,
+                         int n_src, int x_dtype, int64_t k, int layout, int8_t* packed,
+                         float* scales, hipStream_t stream);
+
+/*
  * Raw int32 accumulators acc[m, n] = sum_k xq[m, k] * wq[n, k]: the
  * `flat @ qweight_cpu.transpose(0, 1)` of integer_linear_per_output_reference
  * (w8a8.py:131-133) and QuantizedLinearTensors.integer_golden

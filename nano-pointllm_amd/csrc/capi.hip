@@ -537,6 +537,44 @@ int w8a8_pack_rows(const int8_t* src, int64_t rows, int64_t k, int64_t ld, int l
   return status_of(launch_pack_rows(src, rows, k, ld, layout, packed, stream));
 }
 
+int w8a8_quant_pack_rows(const void* const* x, const int64_t* x_rows, const int64_t* ldx, int n_src,
+                         int x_dtype, int64_t k, int layout, int8_t* packed, float* scales,
+                         hipStream_t stream) {
+  if (n_src < 1 || n_src > kPackSources || k < 0 || k >= (int64_t{1} << 28)) return W8A8_ERR_SHAPE;
+  if (!float_dtype(x_dtype)) return W8A8_ERR_DTYPE;
+  if (layout != W8A8_ROWS_AS_IS && layout != W8A8_ROWS_INTERLEAVE_HALVES) return W8A8_ERR_DTYPE;
+  if (x == nullptr || x_rows == nullptr || ldx == nullptr) return W8A8_ERR_NULL;
+  const bool interleave = layout == W8A8_ROWS_INTERLEAVE_HALVES;
+  int64_t rows = 0;
+  for (int i = 0; i < n_src; ++i) {
+    if (x_rows[i] < 0 || x_rows[i] > kMaxRows - rows || ldx[i] < k) return W8A8_ERR_SHAPE;
+    rows += x_rows[i];
+  }
+  if (interleave && (n_src > 2 || rows % 2 != 0 || (n_src == 2 && x_rows[0] != x_rows[1])))
+    return W8A8_ERR_SHAPE;
+  if (rows == 0 || k == 0) return W8A8_OK;
+  const int64_t es = elem_size(x_dtype);
+  const void* src[kPackSources];
+  int64_t n_rows[kPackSources], ld[kPackSources];
+  for (int i = 0; i < n_src; ++i) {
+    if (x[i] == nullptr && x_rows[i] > 0) return W8A8_ERR_NULL;
+    if (!aligned(x[i], static_cast<uintptr_t>(es))) return W8A8_ERR_ALIGN;
+    src[i] = x[i];
+    n_rows[i] = x_rows[i];
+    ld[i] = ldx[i];
+  }
+  if (packed == nullptr || scales == nullptr) return W8A8_ERR_NULL;
+  if (!aligned(packed, 16) || !aligned(scales, 4)) return W8A8_ERR_ALIGN;
+  if (interleave && n_src == 1) {  // one [gate; up] matrix: its halves
+    n_rows[0] = n_rows[1] = rows / 2;
+    src[1] = static_cast<const char*>(x[0]) + rows / 2 * ldx[0] * es;
+    ld[1] = ldx[0];
+    n_src = 2;
+  }
+  return status_of(launch_quant_pack_rows(src, ld, n_rows, n_src, x_dtype, k, interleave, packed,
+                                          scales, stream));
+}
+
 int w8a8_gemm_i32(const int8_t* xq, int64_t ldq, const int8_t* w_packed, int32_t* acc,
                   int64_t ldacc, int64_t m, int64_t n, int64_t k, void* workspace,
                   int64_t workspace_bytes, hipStream_t stream) {

@@ -475,6 +475,161 @@ __global__ __launch_bounds__(256) void pack_rows_kernel(const int8_t* __restrict
   reinterpret_cast<u32x4*>(dst)[slot] = out;
 }
 
+// Weight rows of up to kPackSources row-major matrices, in packed row order:
+// one after another, or (interleave) packed row p from row p / 2 of matrix
+// p % 2 (the gate/up order of pack_rows_kernel's layout 1).
+struct QuantPackSrc {
+  const void* x[kPackSources];
+  int64_t ld[kPackSources];
+  int64_t end[kPackSources];  // rows of this matrix and those before it
+  int interleave;
+  int vec;  // 16-byte aligned rows, K % 8 == 0
+};
+
+// Per-output weight quantization straight into the packed tiles: one
+// workgroup per 16-row tile block, one wavefront per row.  The row stays in
+// REG 16-byte chunks per lane (as stored, so 16-bit weights take 4 registers
+// per 8 columns) between the absmax and the quantization; REG 0 reads it
+// twice, and takes unaligned rows too.  Every pass of 1024 columns goes through LDS, so that each wavefront
+// writes one whole 1 KiB tile: a row's own 8-byte pieces lie 256 bytes apart
+// in the tiles, and rows on different XCDs would write every line in parts.
+// The LDS copy of a 256-byte tile quarter is padded by 16 bytes: a
+// wavefront's 64 pieces of one row then spread over all banks.  Bound: HBM
+// (2 bytes in, 1 out per 16-bit weight): gate and up of 11008 x 4096 binary16
+// take 56 us with the call, 4.8 TB/s; concatenating them (136 us), quantizing
+// rows (46), packing (33) and interleaving the scales (5) took 215.
+template <typename TX, int REG>
+__global__ __launch_bounds__(1024) void quant_pack_rows_kernel(QuantPackSrc src, int64_t rows,
+                                                               int64_t K, int KB,
+                                                               int8_t* __restrict__ dst,
+                                                               float* __restrict__ scales) {
+  constexpr int kWords = static_cast<int>(sizeof(TX)) / 2;  // 16-byte loads per 8 columns
+  constexpr int kQuarter = 256 + 16;
+  constexpr int kPassTiles = 16;
+  __shared__ u32x4 buf[2][kPassTiles * 4 * kQuarter / 16];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t prow = static_cast<int64_t>(blockIdx.x) * 16 + wave;
+  const bool live = prow < rows;
+  int m = 0;
+  int64_t srow = 0;
+  if (live) {
+    if (src.interleave) {
+      m = static_cast<int>(prow & 1);
+      srow = prow >> 1;
+    } else {
+      while (prow >= src.end[m]) ++m;
+      srow = prow - (m > 0 ? src.end[m - 1] : 0);
+    }
+  }
+  const TX* xr = live ? static_cast<const TX*>(src.x[m]) + srow * src.ld[m] : nullptr;
+  const __amdgpu_buffer_rsrc_t rs = raw_rsrc(xr, static_cast<int>(K * sizeof(TX)));
+  // Chunk c of the lane: columns 8 (64 c + lane), zeros past K.
+  auto fetch_vec = [&](int c, u32x4(&raw)[kWords]) {
+    const int off = (c * 64 + lane) * 8 * static_cast<int>(sizeof(TX));
+#pragma unroll
+    for (int w = 0; w < kWords; ++w) raw[w] = load16(rs, off + 16 * w);
+  };
+  auto fetch_elems = [&](int c, u32x4(&raw)[kWords]) {
+    const int64_t k0 = (static_cast<int64_t>(c) * 64 + lane) * 8;
+    const int64_t left = live ? K - k0 : 0;
+#pragma unroll
+    for (int w = 0; w < kWords; ++w) raw[w] = u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      if (j < left) {
+        if constexpr (sizeof(TX) == 4) {
+          raw[j >> 2][j & 3] = __builtin_bit_cast(uint32_t, xr[k0 + j]);
+        } else {
+          raw[0][j >> 1] |= static_cast<uint32_t>(__builtin_bit_cast(uint16_t, xr[k0 + j]))
+                            << (16 * (j & 1));
+        }
+      }
+    }
+  };
+  auto fetch = [&](int c, u32x4(&raw)[kWords]) {
+    if (src.vec) fetch_vec(c, raw); else fetch_elems(c, raw);
+  };
+  auto elem = [&](const u32x4(&raw)[kWords], int j) {
+    if constexpr (sizeof(TX) == 4) {
+      return __uint_as_float(raw[j >> 2][j & 3]);
+    } else {
+      const uint32_t w = raw[0][j >> 1];
+      return bits_to_f32<TX>(j & 1 ? w >> 16 : w & 0xffffu);
+    }
+  };
+  const int chunks = (KB + 7) / 8;
+  u32x4 v[REG > 0 ? REG : 1][kWords];
+  float amax = 0.0f;
+  auto max_of = [&](const u32x4(&raw)[kWords]) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(elem(raw, j)));
+  };
+  if constexpr (REG > 0) {
+#pragma unroll
+    for (int c = 0; c < REG; ++c) fetch_vec(c, v[c]);
+#pragma unroll
+    for (int c = 0; c < REG; ++c) {
+      max_of(v[c]);
+      // Opaque to the compiler from here, so that it converts the elements
+      // again instead of keeping 8 binary32 values a chunk.
+#pragma unroll
+      for (int w = 0; w < kWords; ++w) asm volatile("" : "+v"(v[c][w]));
+    }
+  } else {
+    for (int c = 0; c < chunks; ++c) {
+      fetch(c, v[0]);
+      max_of(v[0]);
+    }
+  }
+  const float s = scale_from_absmax(wave_max_abs(amax));
+  const float r = 1.0f / s;
+  if (live && lane == 0) scales[prow] = s;
+
+  int8_t* const out = dst + static_cast<int64_t>(blockIdx.x) * KB * kTileBytes;
+  auto put = [&](const u32x4(&raw)[kWords], int half, int8_t* lds) {
+    int32_t qi[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) qi[j] = quant_elem<TX>(elem(raw, j), s, r, true);
+    // Tile 8 half + lane / 8 of the pass, quarter (lane % 8) / 2, slot of row `wave`.
+    *reinterpret_cast<u32x2*>(lds + ((8 * half + (lane >> 3)) * 4 + ((lane & 7) >> 1)) * kQuarter +
+                              wave * 16 + (lane & 1) * 8) =
+        u32x2{pack4_i8(qi[0], qi[1], qi[2], qi[3]), pack4_i8(qi[4], qi[5], qi[6], qi[7])};
+  };
+  // Pass i: columns [1024 i, 1024 i + 1024).  Two LDS buffers: a wavefront
+  // that fills pass i + 2's has passed barrier i + 1, behind every read of
+  // pass i.
+  auto flush = [&](int i, const int8_t* lds) {
+    __syncthreads();
+    const int kb = i * kPassTiles + wave;
+    if (kb < KB)
+      *reinterpret_cast<u32x4*>(out + static_cast<int64_t>(kb) * kTileBytes + lane * 16) =
+          *reinterpret_cast<const u32x4*>(lds + (wave * 4 + (lane >> 4)) * kQuarter + (lane & 15) * 16);
+  };
+  if constexpr (REG > 0) {
+    static_assert(REG % 2 == 0, "a pass takes two chunks");
+#pragma unroll
+    for (int i = 0; i < REG / 2; ++i) {
+      if (2 * i < chunks) {
+        int8_t* lds = reinterpret_cast<int8_t*>(buf[i & 1]);
+        put(v[2 * i], 0, lds);
+        put(v[2 * i + 1], 1, lds);
+        flush(i, lds);
+      }
+    }
+  } else {
+    for (int i = 0; 2 * i < chunks; ++i) {
+      int8_t* lds = reinterpret_cast<int8_t*>(buf[i & 1]);
+      u32x4 second[kWords];
+      fetch(2 * i, v[0]);
+      fetch(2 * i + 1, second);
+      put(v[0], 0, lds);
+      put(second, 1, lds);
+      flush(i, lds);
+    }
+  }
+}
+
 // Row-major int8 copy [rows, K] -> [rows, ldd] with zero columns K..ldd-1.
 // One thread per 16-byte destination chunk.
 __global__ __launch_bounds__(256) void pad_rows_kernel(const int8_t* __restrict__ src,
@@ -607,6 +762,31 @@ hipError_t launch_quant_rows(const void* x, int x_dtype, int64_t ldx, int64_t ro
     default:
       return hipErrorInvalidValue;
   }
+}
+
+// Register chunks per lane: aligned rows of up to 512 REG columns are read once.
+template <typename TX>
+hipError_t quant_pack_dispatch(const QuantPackSrc& src, int64_t rows, int64_t K, int8_t* dst,
+                               float* scales, hipStream_t st) {
+  const int64_t KB = ceil_div(K, kTileK);
+  const dim3 g(static_cast<unsigned>(ceil_div(rows, kTileRows)));
+#define W8A8_QUANT_PACK(R)                                                                     \
+  hipLaunchKernelGGL((quant_pack_rows_kernel<TX, R>), g, dim3(1024), 0, st, src, rows, K,      \
+                     static_cast<int>(KB), dst, scales)
+  if (!src.vec)
+    W8A8_QUANT_PACK(0);
+  else if (K <= 4 * 512)
+    W8A8_QUANT_PACK(4);
+  else if (K <= 8 * 512)
+    W8A8_QUANT_PACK(8);
+  else if (sizeof(TX) == 2 && K <= 16 * 512)
+    W8A8_QUANT_PACK(sizeof(TX) == 2 ? 16 : 0);
+  else if (sizeof(TX) == 2 && K <= 22 * 512)
+    W8A8_QUANT_PACK(sizeof(TX) == 2 ? 22 : 0);
+  else
+    W8A8_QUANT_PACK(0);
+#undef W8A8_QUANT_PACK
+  return hipGetLastError();
 }
 
 template <typename TX, int NT>
@@ -749,6 +929,33 @@ hipError_t launch_qdq_rows(const void* x, int x_dtype, int64_t ldx, int64_t rows
     case kBF16:
       return qdq_dispatch(static_cast<const __hip_bfloat16*>(x), ldx, rows, K, group, out,
                           scales_out, st);
+    default:
+      return hipErrorInvalidValue;
+  }
+}
+
+hipError_t launch_quant_pack_rows(const void* const* x, const int64_t* ld, const int64_t* x_rows,
+                                  int n_src, int x_dtype, int64_t K, bool interleave, int8_t* dst,
+                                  float* scales, hipStream_t st) {
+  QuantPackSrc src{};
+  src.interleave = interleave ? 1 : 0;
+  src.vec = K % 8 == 0;
+  const int64_t per16 = x_dtype == kF32 ? 4 : 8;  // elements of 16 bytes
+  int64_t rows = 0;
+  for (int i = 0; i < n_src; ++i) {
+    rows += x_rows[i];
+    src.x[i] = x[i];
+    src.ld[i] = ld[i];
+    src.end[i] = rows;
+    if (x_rows[i] > 0 && (!aligned16(x[i]) || ld[i] % per16 != 0)) src.vec = 0;
+  }
+  switch (x_dtype) {
+    case kF32:
+      return quant_pack_dispatch<float>(src, rows, K, dst, scales, st);
+    case kF16:
+      return quant_pack_dispatch<__half>(src, rows, K, dst, scales, st);
+    case kBF16:
+      return quant_pack_dispatch<__hip_bfloat16>(src, rows, K, dst, scales, st);
     default:
       return hipErrorInvalidValue;
   }

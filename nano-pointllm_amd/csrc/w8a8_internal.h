@@ -114,6 +114,15 @@ hipError_t launch_qdq_rows(const void* x, int x_dtype, int64_t ldx, int64_t rows
                            int64_t group, int8_t* q, int64_t ldq, void* deq, int64_t ldd,
                            float* scales_out, hipStream_t st);
 
+// Per-row quantization of n_src (1 .. kPackSources) row-major matrices x[i]
+// [x_rows[i], K] (leading dimensions ld) straight into the packed tiles, in
+// order or (interleave, two matrices of equal rows) alternating rows; scales
+// in packed row order.  Rows > 0 in all, K > 0, K * elem < 2^31.
+constexpr int kPackSources = 3;
+hipError_t launch_quant_pack_rows(const void* const* x, const int64_t* ld, const int64_t* x_rows,
+                                  int n_src, int x_dtype, int64_t K, bool interleave, int8_t* dst,
+                                  float* scales, hipStream_t st);
+
 hipError_t launch_pack_rows(const int8_t* src, int64_t rows, int64_t K, int64_t ld, int layout,
                             int8_t* dst, hipStream_t st);
 

@@ -49,6 +49,7 @@ EXPORTED_SYMBOLS = (
     "w8a8_qdq_rows",
     "w8a8_quant_rows_scaled",
     "w8a8_pack_rows",
+    "w8a8_quant_pack_rows",
     "w8a8_gemm_i32",
     "w8a8_linear",
     "w8a8_linear_noalloc",
@@ -86,6 +87,7 @@ _SIGNATURES = {
     "w8a8_qdq_rows": (_int, [_vp, _int, _i64, _i64, _i64, _i64, _vp, _i64, _vp, _i64, _vp, _vp]),
     "w8a8_quant_rows_scaled": (_int, [_vp, _int, _i64, _i64, _i64, _vp, _i64, _vp, _i64, _vp]),
     "w8a8_pack_rows": (_int, [_vp, _i64, _i64, _i64, _int, _vp, _vp]),
+    "w8a8_quant_pack_rows": (_int, [_vp, _vp, _vp, _int, _int, _i64, _int, _vp, _vp, _vp]),
     "w8a8_gemm_i32": (_int, [_vp, _i64, _vp, _vp, _i64, _i64, _i64, _i64, _vp, _i64, _vp]),
     "w8a8_linear": (_int, [_vp, _int, _i64, _vp, _vp, _vp, _int, _vp, _int, _i64, _f32, _int,
                            _i64, _i64, _i64, _vp, _vp, _i64, _vp]),

@@ -74,11 +74,39 @@ class PackedW8A8Weight:
     def from_float(cls, weight: torch.Tensor, bias: torch.Tensor | None = None, *,
                    layout: int = _lib.ROWS_AS_IS) -> "PackedW8A8Weight":
         """Quantize per output row (``per_output_weight_qdq``) and pack."""
-        q, s = _w.quant_rows(weight.detach())
-        return cls.from_int8(q, s, bias, layout=layout)
+        return cls.from_parts([weight], bias, layout=layout)
+
+    @classmethod
+    def from_parts(cls, weights: list[torch.Tensor], bias: torch.Tensor | None = None, *,
+                   layout: int = _lib.ROWS_AS_IS) -> "PackedW8A8Weight":
+        """:meth:`from_float` of the matrices concatenated by rows, quantized
+        straight into the packed tiles by one kernel.  Matrices that it does
+        not take (mixed types or devices, empty or unequal halves) are
+        concatenated and go through int8 rows."""
+        weights = [w.detach() for w in weights]
+        first = weights[0]
+        n = sum(w.shape[0] for w in weights)
+        halves = len(weights) == 1 or (len(weights) == 2
+                                       and first.shape[0] == weights[1].shape[0])
+        if not (0 < len(weights) <= 3 and first.dim() == 2 and first.numel()
+                and all(w.dim() == 2 and w.shape[1] == first.shape[1] and w.dtype == first.dtype
+                        and w.device == first.device for w in weights)
+                and (layout == _lib.ROWS_AS_IS or (n % 2 == 0 and halves))):
+            q, s = _w.quant_rows(first if len(weights) == 1 else torch.cat(weights, dim=0))
+            return cls.from_int8(q, s, bias, layout=layout)
+        device = _lib.require_cuda(*weights, bias)
+        packed, s = _w.quant_pack_rows(weights, layout)
+        b = None if bias is None else bias.detach().to(device=device, dtype=torch.float32).reshape(-1)
+        if b is not None:
+            if b.numel() != n:
+                raise ValueError("scale/bias must have one value per output")
+            if layout == _lib.ROWS_INTERLEAVE_HALVES:
+                b = _interleave_halves(b)
+            b = b.contiguous()
+        return cls(packed, s, b, n, first.shape[1], layout)
 
 
-def _packed(build, source: torch.Tensor, weight_cache, cache_key: str, verify_source: bool,
+def _packed(build, source: torch.Tensor | None, weight_cache, cache_key: str, verify_source: bool,
             layout: int = _lib.ROWS_AS_IS):
     if weight_cache is None:
         return build()
@@ -205,14 +233,16 @@ class W8A8PackedQKV(nn.Module):
                  cache_key: str = "packed_qkv", verify_source: bool = False) -> None:
         super().__init__()
         parts = [_linear_parts(m) for m in (q_proj, k_proj, v_proj)]
-        weight = torch.cat([w for w, _ in parts], dim=0)
+        # The concatenated weight is needed only for its digest in the cache.
+        weight = None if weight_cache is None else torch.cat([w for w, _ in parts], dim=0)
         if all(b is None for _, b in parts):
             bias = None
         else:
             bias = torch.cat([b if b is not None else w.new_zeros(w.shape[0])
                               for w, b in parts], dim=0)
-        self.linear = W8A8Linear(_packed(lambda: PackedW8A8Weight.from_float(weight, bias),
-                                         weight, weight_cache, cache_key, verify_source))
+        self.linear = W8A8Linear(_packed(
+            lambda: PackedW8A8Weight.from_parts([w for w, _ in parts], bias), weight, weight_cache,
+            cache_key, verify_source))
         self.num_heads = num_heads
         self.num_kv_heads = num_kv_heads
         self.head_dim = head_dim
@@ -290,14 +320,15 @@ class W8A8GateUpSiluMul(nn.Module):
                  cache_key: str = "packed_gate_up", verify_source: bool = False) -> None:
         super().__init__()
         (wg, bg), (wu, bu) = _linear_parts(gate_proj), _linear_parts(up_proj)
-        weight = torch.cat([wg, wu], dim=0)
+        weight = None if weight_cache is None else torch.cat([wg, wu], dim=0)
         if bg is None and bu is None:
             bias = None
         else:
             bias = torch.cat([bg if bg is not None else wg.new_zeros(wg.shape[0]),
                               bu if bu is not None else wu.new_zeros(wu.shape[0])])
         self.weight_q = _packed(
-            lambda: PackedW8A8Weight.from_float(weight, bias, layout=_lib.ROWS_INTERLEAVE_HALVES),
+            lambda: PackedW8A8Weight.from_parts([wg, wu], bias,
+                                                layout=_lib.ROWS_INTERLEAVE_HALVES),
             weight, weight_cache, cache_key, verify_source, _lib.ROWS_INTERLEAVE_HALVES)
         self.intermediate = wg.shape[0]
 

@@ -8,6 +8,7 @@ for device memory, reshapes and the static QDQ's elementwise ``q * s``.
 """
 from __future__ import annotations
 
+import ctypes
 from dataclasses import asdict, dataclass
 from functools import lru_cache
 from typing import Any, NamedTuple
@@ -137,6 +138,29 @@ def pack_rows(q: torch.Tensor, layout: int = _lib.ROWS_AS_IS) -> torch.Tensor:
                                       layout, out.data_ptr(), _lib.stream_handle(device)),
                    "w8a8_pack_rows")
     return out
+
+
+def quant_pack_rows(weights: list[torch.Tensor], layout: int = _lib.ROWS_AS_IS
+                    ) -> tuple[torch.Tensor, torch.Tensor]:
+    """Quantize the rows of one to three [rows, K] matrices of one 16/32-bit
+    type (``per_output_weight_qdq``'s integer part) straight into packed
+    tiles: ``(packed int8, f32 scales)``, the scales in packed row order."""
+    device = _lib.require_cuda(*weights)
+    k = weights[0].shape[-1]
+    if any(w.dim() != 2 or w.shape[1] != k or w.dtype != weights[0].dtype for w in weights):
+        raise ValueError("quant_pack_rows expects 2-D matrices of one type and width")
+    views = [_rows_view(w) for w in weights]
+    n = len(views)
+    rows = (ctypes.c_int64 * n)(*[v.shape[0] for v, _ in views])
+    total = sum(rows)
+    packed = torch.empty((packed_bytes(total, k),), dtype=torch.int8, device=device)
+    scales = torch.empty((total,), dtype=torch.float32, device=device)
+    _lib.check(_lib.load().w8a8_quant_pack_rows(
+        (ctypes.c_void_p * n)(*[v.data_ptr() for v, _ in views]), rows,
+        (ctypes.c_int64 * n)(*[ld for _, ld in views]), n, _lib.dtype_code(weights[0].dtype), k,
+        layout, packed.data_ptr(), scales.data_ptr(), _lib.stream_handle(device)),
+        "w8a8_quant_pack_rows")
+    return packed, scales
 
 
 def _workspace(m: int, k: int, device: torch.device) -> torch.Tensor:
