@@ -64,8 +64,9 @@ constexpr int kXcds = 8;
 
 typedef __attribute__((address_space(3))) void lds_void;
 
-// C layout: lane l, register r holds row 4(l/16) + r (activation) and column
-// l%16 (weight row) of the 16x16 block.
+// C layout: lane l, register r holds row 4(l/16) + r of the first operand and
+// row l%16 of the second.  The kernels pass the weights first, so a lane holds
+// four consecutive outputs of one activation row.
 __device__ inline i32x4 mfma_16x16x64(i32x4 a, i32x4 b, i32x4 c) {
   return __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, c, 0, 0, 0);
 }
@@ -84,154 +85,246 @@ __device__ inline void wait_vmcnt() {
 // overtake them; unlike __syncthreads it does not drain outstanding loads.
 __device__ inline void ring_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
+// N consecutive elements as one LDS or global access.
+template <typename T, int N>
+struct alignas(sizeof(T) * N) Pack {
+  T v[N];
+};
+
+// The epilogue's operands of one workgroup tile in LDS: row scales and, per
+// column, the weight scale and bias (or the integer requant's multiplier,
+// shift and bias).  Copied by LDS-DMA before the first operand fragments, so
+// they have landed with them and the epilogue waits for no memory access.
+// Addresses past the operands are clamped to their last element.
+template <int EPI, int BM, int BN>
+struct TileScales {
+  static constexpr bool kRows = EPI != kEpiI32 && EPI != kEpiRequant;
+  static constexpr int kCols = EPI == kEpiI32       ? 0
+                               : EPI == kEpiRequant ? 3
+                                                    : (EPI == kEpiBf16Exact ? 1 : 2);
+  static constexpr int kRowsPad = kRows ? (BM + 63) / 64 * 64 : 4;
+  static constexpr int kColsPad = (BN + 63) / 64 * 64;
+  alignas(16) float sx[kRowsPad];
+  alignas(16) float col[kCols > 0 ? kCols : 1][kCols > 0 ? kColsPad : 4];
+
+  // Called by every wavefront of the workgroup before its first ring load.
+  template <int NW>
+  __device__ inline void load(const GemmParams& p, int mb0, int nb0, int wave, int lane) {
+    auto copy = [&](float* dst, const void* src, int64_t first, int64_t last) {
+      int64_t i = first + lane;
+      i = i < last ? i : last;
+      __builtin_amdgcn_global_load_lds(static_cast<const float*>(src) + i, (lds_void*)dst, 4, 0, 0);
+    };
+    if constexpr (kRows) {
+      for (int c = wave; c < kRowsPad / 64; c += NW)
+        copy(sx + 64 * c, p.sx, static_cast<int64_t>(mb0) * 16 + 64 * c, p.M - 1);
+    }
+    if constexpr (kCols > 0) {
+      // Wavefronts from the last on, so that few hold both kinds of copies.
+      for (int c = NW - 1 - wave; c < kCols * kColsPad / 64; c += NW) {
+        const int k = c / (kColsPad / 64);
+        float* const dst = &col[0][0] + 64 * c;
+        const void* src = p.sw;
+        if constexpr (EPI == kEpiRequant) {
+          src = k == 0 ? static_cast<const void*>(p.rq_mult)
+                       : (k == 1 ? static_cast<const void*>(p.rq_shift) : p.rq_bias);
+        } else if (k == 1) {
+          src = p.bias;
+        }
+        if (src != nullptr) {
+          copy(dst, src, static_cast<int64_t>(nb0) * 16 + 64 * (c % (kColsPad / 64)), p.N - 1);
+        } else {
+          // No bias: -0 changes no binary32 value it is added to, the zeros'
+          // signs included.
+          dst[lane] = EPI == kEpiRequant ? 0.0f : -0.0f;
+        }
+      }
+    }
+  }
+};
+
 // Stores a workgroup's output tile through the epilogue EPI: a WM x WN grid
 // of wavefronts, each holding BR x BC 16x16 blocks of int32 accumulators.
-// Register r of block (i, j) in lane l holds tile row 16(wm BR + i) +
-// 4(l/16) + r and tile column 16(wn BC + j) + l%16.  When the output tile
-// fits in the STAGE_BYTES of LDS at `stage` (whose operand reads every wave
-// has finished once the first barrier below passes), the values go to LDS
-// first and leave as 16-byte row chunks (stored directly, 16 lanes cover only
-// 16 columns of a row: short partial-line writes).
+// Register r of block (i, j) in lane l holds tile row 16(wm BR + i) + l%16
+// and tile column 16(wn BC + j) + 4(l/16) + r: four consecutive columns of one
+// row (the weights are the MFMA's first operand).  A lane therefore needs one
+// row scale per i and four column scales per j (from LDS, TileScales), and
+// packs its four (or with SiLU, whose gate/up pairs are adjacent columns, two)
+// outputs itself.
+//
+// 32-bit outputs leave as 16-byte stores.  16- and 8-bit outputs pass through
+// the operand ring's LDS at `stage` and leave as 16-byte chunks of whole tile
+// rows, in passes of as many row blocks per wavefront as STAGE_BYTES hold.
+// The LDS row stride is an odd multiple of 16 bytes: the 16 rows a wavefront
+// writes at once then start in different banks.
+//
+// Bound by VALU work and stores: 12 thousand shader cycles for a 256 x 256
+// binary16 tile of 8 wavefronts, 5.6 for 128 x 256, 25 with SiLU on 256 x 256.
+// With a row per register instead (a row scale per accumulator, each loaded
+// from memory behind a bounds check, and 2-byte LDS writes) these took 32,
+// 16.6 and 47.  A 2048 x 22016 x 4096 SiLU product went from 191 to 177 us.
 template <int WM, int WN, int BR, int BC, int STAGE_BYTES, int EPI, typename TY, typename TH>
 __device__ inline void store_tile(const GemmParams& p, i32x4 (&acc)[BR][BC], int wm, int wn,
-                                  int mb0, int nb0, int lane, void* stage) {
-  constexpr int BM = 16 * WM * BR;
+                                  int mb0, int nb0, int lane, void* stage,
+                                  const TileScales<EPI, 16 * WM * BR, 16 * WN * BC>& ts) {
+  using Scales = TileScales<EPI, 16 * WM * BR, 16 * WN * BC>;
   constexpr int BN = 16 * WN * BC;
   constexpr bool kHalfCols = EPI == kEpiSilu || EPI == kEpiSiluQ8;  // one output per gate/up pair
+  constexpr int OW = kHalfCols ? 2 : 4;                             // outputs per lane and block
   constexpr int BNO = kHalfCols ? BN / 2 : BN;
   constexpr int kOutBytes = static_cast<int>(sizeof(TY));
-  constexpr bool kStage = BM * BNO * kOutBytes <= STAGE_BYTES && (BNO * kOutBytes) % 16 == 0;
-  [[maybe_unused]] TY* const stile = static_cast<TY*>(stage);
-  if constexpr (kStage) ring_barrier();  // every wave is done reading the ring
-  // Writes output (m, n_out) of tile-local row ml and column nlo.
-  auto put = [&](int ml, int nlo, bool ok, int64_t m, int64_t n_out, TY v) {
-    if constexpr (kStage) {
-      stile[ml * BNO + nlo] = v;
-    } else {
-      if (ok) static_cast<TY*>(p.y)[m * p.ldy + n_out] = v;
-    }
+  constexpr bool kStage = kOutBytes < 4;
+  constexpr int kRowBytes = BNO * kOutBytes;
+  constexpr int kStride = (kRowBytes / 16 | 1) * 16;
+  static_assert(kRowBytes % 16 == 0, "tile rows are whole 16-byte chunks");
+  constexpr int kFit = STAGE_BYTES / (WM * 16 * kStride);
+  constexpr int IPP = !kStage || kFit > BR ? BR : kFit;  // row blocks per wavefront and pass
+  static_assert(IPP >= 1, "a pass holds at least one row block per wavefront");
+
+  const int quad = lane >> 4;
+  const int64_t m0 = static_cast<int64_t>(mb0) * 16;
+  const int64_t n0 = static_cast<int64_t>(nb0) * 16;
+  // This lane's row of block i and first column of block j, in the tile.
+  auto row_of = [&](int i) { return 16 * (wm * BR + i) + (lane & 15); };
+  auto col_of = [&](int j) { return 16 * (wn * BC + j) + 4 * quad; };
+
+  [[maybe_unused]] float sx[BR];
+  if constexpr (Scales::kRows) {
+#pragma unroll
+    for (int i = 0; i < BR; ++i) sx[i] = ts.sx[row_of(i)];
+  }
+  // Column operands k of block column j.
+  auto cols = [&](int k, int j) __attribute__((always_inline)) {
+    return *reinterpret_cast<const Pack<float, 4>*>(&ts.col[k][col_of(j)]);
   };
+  struct Cols {
+    Pack<float, 4> c[Scales::kCols > 0 ? Scales::kCols : 1];
+  };
+  auto cols_of = [&](int j) __attribute__((always_inline)) {
+    Cols c;
+    if constexpr (Scales::kCols > 0) {
 #pragma unroll
-  for (int i = 0; i < BR; ++i)
-#pragma unroll
-  for (int j = 0; j < BC; ++j) {
-    const int nl = 16 * (wn * BC + j) + (lane & 15);
-    const int64_t n = static_cast<int64_t>(nb0) * 16 + nl;
-    const bool n_ok = n < p.N;
-    float swn = 0.0f;
-    if constexpr (EPI != kEpiI32 && EPI != kEpiRequant) swn = n_ok ? p.sw[n] : 0.0f;
-    uint32_t rq_mult = 0;
-    int32_t rq_shift = 0, rq_bias = 0;
-    if constexpr (EPI == kEpiRequant) {
-      if (n_ok) {
-        rq_mult = p.rq_mult[n];
-        rq_shift = p.rq_shift[n];
-        rq_bias = p.rq_bias != nullptr ? p.rq_bias[n] : 0;
-      }
+      for (int k = 0; k < Scales::kCols; ++k) c.c[k] = cols(k, j);
     }
+    return c;
+  };
+
+  // The lane's outputs of block (i, j).
+  auto outputs = [&](int i, int j, const Cols& cj) __attribute__((always_inline)) {
+    Pack<TY, OW> o;
+    const i32x4 a = acc[i][j];
     if constexpr (kHalfCols) {
-      // kEpiSilu with absmax_parts: |h| of this lane's output for row pair r / 2.
-      [[maybe_unused]] float habs[2] = {0.0f, 0.0f};
-      // Interleaved gate/up: even column = gate, odd column = up of output
-      // n / 2.  Every lane dequantizes its own column at rows r and r + 1;
-      // then the even lane forms output row r from its gate and the odd
-      // lane's up, and the odd lane output row r + 1 from the even lane's
-      // gate and its own up, so each SiLU is evaluated by one lane.
-      const bool odd = (lane & 1) != 0;
 #pragma unroll
-      for (int r = 0; r < 4; r += 2) {
-        const int ml0 = 16 * (wm * BR + i) + 4 * (lane >> 4) + r;
-        float v[2];
-        bool vok[2];
+      for (int e = 0; e < 2; ++e) {
+        float gu[2];
 #pragma unroll
-        for (int e = 0; e < 2; ++e) {
-          const int64_t m = static_cast<int64_t>(mb0) * 16 + ml0 + e;
-          const bool m_ok = m < p.M;
-          vok[e] = m_ok && n_ok;
-          const float sxm = m_ok ? p.sx[m] : 0.0f;
-          v[e] = vok[e] ? to_f32(from_f32<TH>(dequant1(acc[i][j][r + e], sxm, swn, p.bias, n)))
-                        : 0.0f;
-        }
-        const float x = __shfl_xor(odd ? v[0] : v[1], 1);
-        const float g = odd ? x : v[0];
-        const float u = odd ? v[1] : x;
-        const int ml = ml0 + (odd ? 1 : 0);
-        const int64_t m = static_cast<int64_t>(mb0) * 16 + ml;
-        const bool ok = odd ? vok[1] : vok[0];
-        const TH h = from_f32<TH>(silu_mul<TH>(g, u));
+        for (int c = 0; c < 2; ++c)
+          gu[c] = to_f32(from_f32<TH>(
+              dequant1b(a[2 * e + c], sx[i], cj.c[0].v[2 * e + c], true, cj.c[1].v[2 * e + c])));
+        const TH h = from_f32<TH>(silu_mul<TH>(gu[0], gu[1]));
         if constexpr (EPI == kEpiSilu) {
-          put(ml, nl / 2, ok, m, n / 2, h);
-          if (ok) habs[r >> 1] = fabsf(to_f32(h));
+          o.v[e] = h;
         } else {
-          put(ml, nl / 2, ok, m, n / 2, static_cast<int8_t>(quant1(to_f32(h), p.out_scale)));
-        }
-      }
-      if constexpr (EPI == kEpiSilu) {
-        if (p.absmax_parts != nullptr) {
-          // Lanes of one parity in a 16-lane group hold the same output row
-          // (even lanes row r, odd lanes row r + 1) over the 8 outputs of
-          // packed block nb: reduce over them, then one store per row.
-          const int64_t nb = static_cast<int64_t>(nb0) + wn * BC + j;
-#pragma unroll
-          for (int h2 = 0; h2 < 2; ++h2) {
-            float v = habs[h2];
-#pragma unroll
-            for (int off = 2; off < 16; off <<= 1) v = fmaxf(v, __shfl_xor(v, off));
-            const int64_t m = static_cast<int64_t>(mb0) * 16 + 16 * (wm * BR + i) +
-                              4 * (lane >> 4) + 2 * h2 + (lane & 1);
-            if ((lane & 15) < 2 && m < p.M && nb < p.NB) p.absmax_parts[m * p.NB + nb] = v;
-          }
+          o.v[e] = static_cast<int8_t>(quant1(to_f32(h), p.out_scale));
         }
       }
     } else {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int ml = 16 * (wm * BR + i) + 4 * (lane >> 4) + r;
-        const int64_t m = static_cast<int64_t>(mb0) * 16 + ml;
-        const bool m_ok = m < p.M;
-        const bool ok = m_ok && n_ok;
-        const int32_t a = acc[i][j][r];
         if constexpr (EPI == kEpiI32) {
-          put(ml, nl, ok, m, n, a);
+          o.v[r] = a[r];
         } else if constexpr (EPI == kEpiDequant) {
-          const float sxm = m_ok ? p.sx[m] : 0.0f;
-          put(ml, nl, ok, m, n, from_f32<TY>(dequant1(a, sxm, swn, ok ? p.bias : nullptr, n)));
+          o.v[r] = from_f32<TY>(dequant1b(a[r], sx[i], cj.c[0].v[r], true, cj.c[1].v[r]));
         } else if constexpr (EPI == kEpiRequant) {
-          put(ml, nl, ok, m, n, static_cast<int8_t>(requant1(a, rq_bias, rq_mult, rq_shift)));
+          o.v[r] = static_cast<int8_t>(requant1(
+              a[r], __builtin_bit_cast(int32_t, cj.c[2].v[r]),
+              __builtin_bit_cast(uint32_t, cj.c[0].v[r]), __builtin_bit_cast(int32_t, cj.c[1].v[r])));
         } else {
           static_assert(EPI == kEpiBf16Exact, "epilogue");
-          const float sxm = m_ok ? p.sx[m] : 0.0f;
-          put(ml, nl, ok, m, n,
-              __builtin_bit_cast(TY, dequant_bf16_exact(a, f16_bits(sxm), f16_bits(swn))));
+          o.v[r] = __builtin_bit_cast(
+              TY, dequant_bf16_exact(a[r], f16_bits(sx[i]), f16_bits(cj.c[0].v[r])));
         }
       }
     }
-  }
-  if constexpr (kStage) {
-    __syncthreads();
-    constexpr int EV = 16 / kOutBytes;  // outputs per 16-byte chunk
-    constexpr int CPR = BNO / EV;       // chunks per tile row
-    constexpr int NT = WM * WN * 64;
-    constexpr int RPP = NT / CPR;       // tile rows per pass; threads past RPP * CPR idle
-    static_assert(RPP >= 1, "a pass covers at least one tile row");
-    const int64_t n_out_total = kHalfCols ? p.N / 2 : p.N;
-    const int64_t n0 = kHalfCols ? static_cast<int64_t>(nb0) * 8 : static_cast<int64_t>(nb0) * 16;
-    const bool vec_ok =
-        ((reinterpret_cast<uintptr_t>(p.y) | static_cast<uintptr_t>(p.ldy * kOutBytes)) & 15) == 0;
+    return o;
+  };
+
+  const bool vec_ok =
+      ((reinterpret_cast<uintptr_t>(p.y) | static_cast<uintptr_t>(p.ldy * kOutBytes)) & 15) == 0;
+  if constexpr (!kStage) {
 #pragma unroll
-    for (int base = 0; base < BM; base += RPP) {
-      const int ml = base + static_cast<int>(threadIdx.x) / CPR;
-      const int nlo = (static_cast<int>(threadIdx.x) % CPR) * EV;
-      const int64_t m = static_cast<int64_t>(mb0) * 16 + ml;
-      const int64_t n = n0 + nlo;
-      if (static_cast<int>(threadIdx.x) < RPP * CPR && ml < BM && m < p.M && n < n_out_total) {
-        TY* dst = static_cast<TY*>(p.y) + m * p.ldy + n;
-        const TY* src = stile + ml * BNO + nlo;
-        if (vec_ok && n + EV <= n_out_total) {
-          *reinterpret_cast<i32x4*>(dst) = *reinterpret_cast<const i32x4*>(src);
-        } else {
-          for (int e = 0; e < EV; ++e)
-            if (n + e < n_out_total) dst[e] = src[e];
+    for (int j = 0; j < BC; ++j) {
+      const Cols cj = cols_of(j);
+#pragma unroll
+      for (int i = 0; i < BR; ++i) {
+        const int64_t m = m0 + row_of(i);
+        const int64_t n = n0 + col_of(j);
+        const Pack<TY, 4> o = outputs(i, j, cj);
+        if (m < p.M && n < p.N) {
+          TY* const dst = static_cast<TY*>(p.y) + m * p.ldy + n;
+          if (vec_ok && n + 4 <= p.N) {
+            *reinterpret_cast<Pack<TY, 4>*>(dst) = o;
+          } else {
+            for (int r = 0; r < 4; ++r)
+              if (n + r < p.N) dst[r] = o.v[r];
+          }
+        }
+      }
+    }
+  } else {
+    char* const st = static_cast<char*>(stage);
+    constexpr int EV = 16 / kOutBytes;    // outputs per 16-byte chunk
+    constexpr int CPR = kRowBytes / 16;   // chunks per tile row
+    constexpr int NT = WM * WN * 64;
+    constexpr int RPP = NT / CPR;         // rows per sweep; threads past RPP * CPR idle
+    static_assert(RPP >= 1, "a sweep covers at least one tile row");
+    const int64_t n_out_total = kHalfCols ? p.N / 2 : p.N;
+    const int64_t n0_out = kHalfCols ? n0 / 2 : n0;
+    const int crow = static_cast<int>(threadIdx.x) / CPR;
+    const int cchunk = static_cast<int>(threadIdx.x) % CPR;
+#pragma unroll
+    for (int i0 = 0; i0 < BR; i0 += IPP) {
+      const int ni = BR - i0 < IPP ? BR - i0 : IPP;  // compile-time after unrolling
+      ring_barrier();  // the ring's (or the last pass's) readers are done
+#pragma unroll
+      for (int j = 0; j < BC; ++j) {
+        const Cols cj = cols_of(j);
+#pragma unroll
+        for (int i = i0; i < i0 + ni; ++i) {
+          const Pack<TY, OW> o = outputs(i, j, cj);
+          const int row = 16 * (wm * ni + i - i0) + (lane & 15);
+          const int col = kHalfCols ? col_of(j) / 2 : col_of(j);
+          *reinterpret_cast<Pack<TY, OW>*>(st + row * kStride + col * kOutBytes) = o;
+          if constexpr (EPI == kEpiSilu) {
+            if (p.absmax_parts != nullptr) {
+              // The row's 8 outputs of packed block nb lie in the four lanes
+              // l%16 + 16q.
+              float v = fmaxf(fabsf(to_f32(o.v[0])), fabsf(to_f32(o.v[1])));
+              v = fmaxf(v, __shfl_xor(v, 16));
+              v = fmaxf(v, __shfl_xor(v, 32));
+              const int64_t m = m0 + row_of(i);
+              const int64_t nb = static_cast<int64_t>(nb0) + wn * BC + j;
+              if (quad == 0 && m < p.M && nb < p.NB) p.absmax_parts[m * p.NB + nb] = v;
+            }
+          }
+        }
+      }
+      ring_barrier();
+      const int rows = WM * 16 * ni;
+#pragma unroll
+      for (int base = 0; base < rows; base += RPP) {
+        const int row = base + crow;
+        const int64_t m = m0 + 16 * (row / (16 * ni) * BR + i0) + row % (16 * ni);
+        const int64_t n = n0_out + cchunk * EV;
+        if (crow < RPP && row < rows && m < p.M && n < n_out_total) {
+          TY* const dst = static_cast<TY*>(p.y) + m * p.ldy + n;
+          const TY* const src = reinterpret_cast<const TY*>(st + row * kStride + cchunk * 16);
+          if (vec_ok && n + EV <= n_out_total) {
+            *reinterpret_cast<i32x4*>(dst) = *reinterpret_cast<const i32x4*>(src);
+          } else {
+            for (int e = 0; e < EV; ++e)
+              if (n + e < n_out_total) dst[e] = src[e];
+          }
         }
       }
     }
@@ -255,7 +348,13 @@ __global__ __launch_bounds__(WM * WN * 64, OCC * WM * WN / 4) void gemm_kernel(G
   // Fragment copies per wave per stage: LPW for the first FS - (LPW-1) NW
   // waves, LPW - 1 for the rest.
   constexpr int LPW = (FS + NW - 1) / NW;
-  __shared__ i32x4 lds[STG][FS][64];
+  using Scales = TileScales<EPI, 16 * BMF, 16 * BNF>;
+  constexpr int kRing = STG * FS * 1024;
+  // One array for the ring and the scales: the compiler takes LDS-DMA into
+  // one object to be finished by its own wait before it reads another.
+  __shared__ i32x4 smem[(kRing + sizeof(Scales)) / 16];
+  auto lds = reinterpret_cast<i32x4 (*)[FS][64]>(smem);
+  Scales& scales = *reinterpret_cast<Scales*>(smem + kRing / 16);
 
   // XCD-major tile mapping: workgroup b runs on XCD b % 8.
   const int b = blockIdx.x;
@@ -310,6 +409,8 @@ __global__ __launch_bounds__(WM * WN * 64, OCC * WM * WN / 4) void gemm_kernel(G
 #pragma unroll
       for (int r = 0; r < 4; ++r) acc[i][j][r] = 0;
 
+  scales.template load<NW>(p, mb0, nb0, wave, lane);
+
 #pragma unroll
   for (int s = 0; s < STG - 1; ++s)
     if (s < NS) issue(s, s);
@@ -340,13 +441,12 @@ __global__ __launch_bounds__(WM * WN * 64, OCC * WM * WN / 4) void gemm_kernel(G
 #pragma unroll
         for (int i = 0; i < BR; ++i)
 #pragma unroll
-          for (int j = 0; j < BC; ++j) acc[i][j] = mfma_16x16x64(af[i], bf[j], acc[i][j]);
+          for (int j = 0; j < BC; ++j) acc[i][j] = mfma_16x16x64(bf[j], af[i], acc[i][j]);
       }
     }
   }
 
-  store_tile<WM, WN, BR, BC, STG * FS * 1024, EPI, TY, TH>(p, acc, wm, wn, mb0, nb0, lane,
-                                                           &lds[0][0][0]);
+  store_tile<WM, WN, BR, BC, kRing, EPI, TY, TH>(p, acc, wm, wn, mb0, nb0, lane, smem, scales);
 }
 
 // Workgroup barrier with the wave's LDS reads complete, through the builtin
@@ -403,7 +503,10 @@ __global__ __launch_bounds__(NW * 64, NW / 4) void gemm_wd_kernel(GemmParams p) 
   constexpr int kRing = S * A * 1024;
   constexpr int kOut = BM * (kHalfCols ? BN / 2 : BN) * static_cast<int>(sizeof(TY));
   constexpr int kLds = kRing > kOut ? kRing : kOut;
-  __shared__ i32x4 lds[kLds / 16];
+  using Scales = TileScales<EPI, BM, BN>;
+  // One array, as in gemm_kernel.
+  __shared__ i32x4 lds[(kLds + sizeof(Scales)) / 16];
+  Scales& scales = *reinterpret_cast<Scales*>(lds + kLds / 16);
   auto ring = reinterpret_cast<i32x4 (*)[A][64]>(lds);
 
   const int b = blockIdx.x;
@@ -451,6 +554,7 @@ __global__ __launch_bounds__(NW * 64, NW / 4) void gemm_wd_kernel(GemmParams p) 
   constexpr int kLoadsFull = LPW + B;
   constexpr int kLoadsPart = LPW - 1 + B;
 
+  scales.template load<NW>(p, mb0, nb0, wave, lane);
   static_for<D>([&](auto i) __attribute__((always_inline)) {
     if (decltype(i)::value < KB) issue(decltype(i)::value, i);
   });
@@ -488,7 +592,7 @@ __global__ __launch_bounds__(NW * 64, NW / 4) void gemm_wd_kernel(GemmParams p) 
 #pragma unroll
     for (int i = 0; i < A; ++i)
 #pragma unroll
-      for (int j = 0; j < B; ++j) acc[i][j] = mfma_16x16x64(af[cur][i], breg[set][j], acc[i][j]);
+      for (int j = 0; j < B; ++j) acc[i][j] = mfma_16x16x64(breg[set][j], af[cur][i], acc[i][j]);
   };
   // Unrolled by U, a multiple of the register-set count and of 2, so every
   // set and buffer index is static.
@@ -508,7 +612,7 @@ __global__ __launch_bounds__(NW * 64, NW / 4) void gemm_wd_kernel(GemmParams p) 
            std::false_type{});
   });
 
-  store_tile<1, NW, A, B, kLds, EPI, TY, TH>(p, acc, 0, wave, mb0, nb0, lane, lds);
+  store_tile<1, NW, A, B, kLds, EPI, TY, TH>(p, acc, 0, wave, mb0, nb0, lane, lds, scales);
 }
 
 // Launches the weights-direct kernel for the problem in p.
