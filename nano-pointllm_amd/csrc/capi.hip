@@ -184,7 +184,7 @@ inline bool use_gemv(int64_t m, int64_t n, int64_t k) {
 // kernels take the residual-add epilogue (op.res) themselves; the GEMM
 // writes its output first and the add runs over it.
 inline hipError_t run_product(const LinearOperands& op, hipStream_t st) {
-  if (use_gemv(op.M, op.N, op.K)) return launch_gemv(op, st);
+  if (op.a_tiles || use_gemv(op.M, op.N, op.K)) return launch_gemv(op, st);
   if (op.res == nullptr) return launch_gemm(op, st);
   LinearOperands plain = op;
   plain.res = nullptr;
@@ -297,12 +297,13 @@ int linear_impl(const void* x, int x_dtype, int64_t ldx, const int8_t* w_packed,
   float* sx = x_scale_out != nullptr ? x_scale_out : static_cast<float*>(workspace);
   int8_t* act = static_cast<int8_t*>(workspace) + scale_region(m);
   const int64_t kp = round_up(k, kTileK);
-  const bool gemv = use_gemv(m, n, k);
-  hipError_t e = launch_quant_rows(x, x_dtype, ldx, m, k, nullptr, 0, act, kp, kp, !gemv, sx,
-                                   stream);
+  const bool tiles = gemv_tiles_supported(m, n, k, epilogue, y_dtype);
+  hipError_t e = launch_quant_rows(x, x_dtype, ldx, m, k, nullptr, 0, act, kp, kp,
+                                   tiles || !use_gemv(m, n, k), sx, stream);
   if (e != hipSuccess) return status_of(e);
   LinearOperands op = make_ops(act, kp, sx, w_packed, w_scale, bias, epilogue, y, y_dtype, ldy,
                                y_scale, inter_dtype, m, n, k);
+  op.a_tiles = tiles;
   op.absmax_parts = absmax_parts;
   set_residual(op, ra);
   return status_of(run_product(op, stream));

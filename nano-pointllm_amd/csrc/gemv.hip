@@ -57,9 +57,136 @@ __device__ inline i32x4 mfma_16x16x64(i32x4 a, i32x4 b, i32x4 c) {
   return __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, c, 0, 0, 0);
 }
 
+// The operands of the output a thread of gemv_kernel or gemv_tiles_kernel
+// writes first (element e == tid of the workgroup's NBW blocks x MT row tiles),
+// requested before the weights so that the epilogue does not wait a memory
+// round trip for them.  Clamped addresses: the outputs they stand for past M
+// or N are not written.
+template <typename TY>
+struct FirstOutput {
+  TY res{};
+  float sx = 0.0f, sw = 0.0f;
+  template <int MT, int NBW, int EPI>
+  __device__ inline void load(const GemvParams& p, int64_t nb0, int tid) {
+    if constexpr (EPI == kEpiDequant) {
+      const int e = tid < NBW * MT * 256 ? tid : 0;
+      const int m = min(((e % (MT * 256)) >> 8) * 16 + ((e & 255) >> 4), p.M - 1);
+      const int64_t nc = (nb0 + e / (MT * 256)) * 16 + (e & 15);
+      const int64_t n = nc < p.N ? nc : p.N - 1;
+      sx = p.sx[m];
+      sw = p.sw[n];
+      if (p.res != nullptr) res = static_cast<const TY*>(p.res)[m * p.ld_res + n];
+    }
+  }
+};
+
+// Sums the wavefronts' int32 partials red[w][j * 256 MT + 256 mt + 16 row +
+// column] (complete: the caller has passed a barrier) and writes the NBW
+// blocks' outputs through the epilogue EPI.
+template <int WAVES, int MT, int NBW, int EPI, typename TY, typename TH>
+__device__ inline void gemv_store(const GemvParams& p, const int32_t (*red)[NBW * MT * 256],
+                                  int64_t nb0, int tid, const FirstOutput<TY>& first) {
+  constexpr int NT = WAVES * 64;
+  constexpr int TB = MT * 256;  // int32 partials of one block per wave
+  [[maybe_unused]] auto dequant = [&](int32_t s, int e, int m, int64_t n) {
+    const bool f = e == tid;
+    return dequant1(s, f ? first.sx : p.sx[m], f ? first.sw : p.sw[n], p.bias, n);
+  };
+  if constexpr (EPI == kEpiI32 || EPI == kEpiDequant || EPI == kEpiRequant ||
+                EPI == kEpiBf16Exact) {
+    for (int e = tid; e < NBW * TB; e += NT) {
+      const int m = ((e % TB) >> 8) * 16 + ((e & 255) >> 4);
+      const int64_t nb = nb0 + e / TB;
+      const int64_t n = nb * 16 + (e & 15);
+      if constexpr (EPI == kEpiDequant) {
+        if (p.res != nullptr) {
+          // Residual-add epilogue: the chunk sums need every lane, so no lane
+          // leaves before them (NBW * TB and NT are multiples of 64).
+          const bool ok = m < p.M && nb < p.NB && n < p.N;
+          float v = 0.0f;
+          if (ok) {
+            int32_t s = 0;
+#pragma unroll
+            for (int w = 0; w < WAVES; ++w) s += red[w][e];
+            const TY r = e == tid ? first.res : static_cast<const TY*>(p.res)[m * p.ld_res + n];
+            const TY o = add_rounded(from_f32<TY>(dequant(s, e, m, n)), r);
+            static_cast<TY*>(p.y)[static_cast<int64_t>(m) * p.ldy + n] = o;
+            v = to_f32(o);
+          }
+          if (p.ss_parts != nullptr) {
+            const float cs = chunk_sumsq8(v);
+            if ((e & 7) == 0 && ok) p.ss_parts[m * p.ld_parts + (n >> 3)] = cs;
+          }
+          continue;
+        }
+      }
+      if (m >= p.M || nb >= p.NB || n >= p.N) continue;
+      int32_t s = 0;
+#pragma unroll
+      for (int w = 0; w < WAVES; ++w) s += red[w][e];
+      TY* y = static_cast<TY*>(p.y) + static_cast<int64_t>(m) * p.ldy + n;
+      if constexpr (EPI == kEpiI32) {
+        *y = s;
+      } else if constexpr (EPI == kEpiRequant) {
+        *y = static_cast<int8_t>(
+            requant1(s, p.rq_bias != nullptr ? p.rq_bias[n] : 0, p.rq_mult[n], p.rq_shift[n]));
+      } else if constexpr (EPI == kEpiBf16Exact) {
+        *y = __builtin_bit_cast(TY, dequant_bf16_exact(s, f16_bits(p.sx[m]), f16_bits(p.sw[n])));
+      } else {
+        *y = from_f32<TY>(dequant(s, e, m, n));
+      }
+    }
+  } else {
+    // Interleaved gate/up: packed rows 2c (gate) and 2c+1 (up) of this block
+    // produce output column nb*8 + c.
+    const int64_t n_out_total = p.N / 2;
+    // NBW * MT * 128 and NT are multiples of 64, so every wavefront runs the
+    // same trip count and the shuffles below run in uniform control flow.
+    for (int e = tid; e < NBW * MT * 128; e += NT) {
+      const int j = e / (MT * 128);
+      const int mt = (e % (MT * 128)) >> 7;
+      const int i = (e & 127) >> 3;
+      const int c = e & 7;
+      const int m = mt * 16 + i;
+      const int64_t nb = nb0 + j;
+      const int64_t n_out = nb * 8 + c;
+      float habs = 0.0f;
+      if (m < p.M && nb < p.NB && n_out < n_out_total) {
+        const int base = j * TB + mt * 256 + i * 16 + 2 * c;
+        int32_t sg = 0, su = 0;
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) {
+          sg += red[w][base];
+          su += red[w][base + 1];
+        }
+        const int64_t ng = nb * 16 + 2 * c;
+        const float sxm = p.sx[m];
+        const float g = to_f32(from_f32<TH>(dequant1(sg, sxm, p.sw[ng], p.bias, ng)));
+        const float u = to_f32(from_f32<TH>(dequant1(su, sxm, p.sw[ng + 1], p.bias, ng + 1)));
+        const TH h = from_f32<TH>(silu_mul<TH>(g, u));
+        TY* y = static_cast<TY*>(p.y) + static_cast<int64_t>(m) * p.ldy + n_out;
+        if constexpr (EPI == kEpiSilu) {
+          *y = h;
+          habs = fabsf(to_f32(h));
+        } else {
+          *y = static_cast<int8_t>(quant1(to_f32(h), p.out_scale));
+        }
+      }
+      if constexpr (EPI == kEpiSilu) {
+        if (p.absmax_parts != nullptr) {
+          // Row m's 8 outputs of this block sit in 8 consecutive lanes.
+#pragma unroll
+          for (int off = 1; off < 8; off <<= 1) habs = fmaxf(habs, __shfl_xor(habs, off));
+          if (c == 0 && m < p.M && nb < p.NB)
+            p.absmax_parts[static_cast<int64_t>(m) * p.NB + nb] = habs;
+        }
+      }
+    }
+  }
+}
+
 template <int WAVES, int MT, int CH, int NBW, int EPI, typename TY, typename TH>
 __global__ __launch_bounds__(WAVES * 64) void gemv_kernel(GemvParams p) {
-  constexpr int NT = WAVES * 64;
   constexpr int TB = MT * 256;  // int32 partials of one block per wave
   __shared__ int32_t red[WAVES][NBW * TB];
 
@@ -96,18 +223,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_kernel(GemvParams p) {
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) acc[j][mt] = i32x4{0, 0, 0, 0};
 
-  // Residual-add epilogue: the residual of this thread's first output is
-  // requested before the weights, so the epilogue does not wait a memory
-  // round trip for it (later outputs, when a thread has several, load then).
-  [[maybe_unused]] TY res_first{};
-  if constexpr (EPI == kEpiDequant) {
-    if (p.res != nullptr && tid < NBW * TB) {
-      const int m = ((tid % TB) >> 8) * 16 + ((tid & 255) >> 4);
-      const int64_t nb = nb0 + tid / TB;
-      const int64_t n = nb * 16 + (tid & 15);
-      if (m < p.M && nb < p.NB && n < p.N) res_first = static_cast<const TY*>(p.res)[m * p.ld_res + n];
-    }
-  }
+  FirstOutput<TY> first;
+  first.template load<MT, NBW, EPI>(p, nb0, tid);
 
   i32x4 wb0[NBW][CH], wb1[NBW][CH];
   i32x4 ab0[MT][CH], ab1[MT][CH];
@@ -167,97 +284,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_kernel(GemvParams p) {
     }
   __syncthreads();
 
-  if constexpr (EPI == kEpiI32 || EPI == kEpiDequant || EPI == kEpiRequant ||
-                EPI == kEpiBf16Exact) {
-    for (int e = tid; e < NBW * TB; e += NT) {
-      const int m = ((e % TB) >> 8) * 16 + ((e & 255) >> 4);
-      const int64_t nb = nb0 + e / TB;
-      const int64_t n = nb * 16 + (e & 15);
-      if constexpr (EPI == kEpiDequant) {
-        if (p.res != nullptr) {
-          // Residual-add epilogue: the chunk sums need every lane, so no lane
-          // leaves before them (NBW * TB and NT are multiples of 64).
-          const bool ok = m < p.M && nb < p.NB && n < p.N;
-          float v = 0.0f;
-          if (ok) {
-            int32_t s = 0;
-#pragma unroll
-            for (int w = 0; w < WAVES; ++w) s += red[w][e];
-            const TY r = e == tid ? res_first : static_cast<const TY*>(p.res)[m * p.ld_res + n];
-            const TY o = add_rounded(from_f32<TY>(dequant1(s, p.sx[m], p.sw[n], p.bias, n)), r);
-            static_cast<TY*>(p.y)[static_cast<int64_t>(m) * p.ldy + n] = o;
-            v = to_f32(o);
-          }
-          if (p.ss_parts != nullptr) {
-            const float cs = chunk_sumsq8(v);
-            if ((e & 7) == 0 && ok) p.ss_parts[m * p.ld_parts + (n >> 3)] = cs;
-          }
-          continue;
-        }
-      }
-      if (m >= p.M || nb >= p.NB || n >= p.N) continue;
-      int32_t s = 0;
-#pragma unroll
-      for (int w = 0; w < WAVES; ++w) s += red[w][e];
-      TY* y = static_cast<TY*>(p.y) + static_cast<int64_t>(m) * p.ldy + n;
-      if constexpr (EPI == kEpiI32) {
-        *y = s;
-      } else if constexpr (EPI == kEpiRequant) {
-        *y = static_cast<int8_t>(
-            requant1(s, p.rq_bias != nullptr ? p.rq_bias[n] : 0, p.rq_mult[n], p.rq_shift[n]));
-      } else if constexpr (EPI == kEpiBf16Exact) {
-        *y = __builtin_bit_cast(TY, dequant_bf16_exact(s, f16_bits(p.sx[m]), f16_bits(p.sw[n])));
-      } else {
-        *y = from_f32<TY>(dequant1(s, p.sx[m], p.sw[n], p.bias, n));
-      }
-    }
-  } else {
-    // Interleaved gate/up: packed rows 2c (gate) and 2c+1 (up) of this block
-    // produce output column nb*8 + c.
-    const int64_t n_out_total = p.N / 2;
-    // NBW * MT * 128 and NT are multiples of 64, so every wavefront runs the
-    // same trip count and the shuffles below run in uniform control flow.
-    for (int e = tid; e < NBW * MT * 128; e += NT) {
-      const int j = e / (MT * 128);
-      const int mt = (e % (MT * 128)) >> 7;
-      const int i = (e & 127) >> 3;
-      const int c = e & 7;
-      const int m = mt * 16 + i;
-      const int64_t nb = nb0 + j;
-      const int64_t n_out = nb * 8 + c;
-      float habs = 0.0f;
-      if (m < p.M && nb < p.NB && n_out < n_out_total) {
-        const int base = j * TB + mt * 256 + i * 16 + 2 * c;
-        int32_t sg = 0, su = 0;
-#pragma unroll
-        for (int w = 0; w < WAVES; ++w) {
-          sg += red[w][base];
-          su += red[w][base + 1];
-        }
-        const int64_t ng = nb * 16 + 2 * c;
-        const float sxm = p.sx[m];
-        const float g = to_f32(from_f32<TH>(dequant1(sg, sxm, p.sw[ng], p.bias, ng)));
-        const float u = to_f32(from_f32<TH>(dequant1(su, sxm, p.sw[ng + 1], p.bias, ng + 1)));
-        const TH h = from_f32<TH>(silu_mul<TH>(g, u));
-        TY* y = static_cast<TY*>(p.y) + static_cast<int64_t>(m) * p.ldy + n_out;
-        if constexpr (EPI == kEpiSilu) {
-          *y = h;
-          habs = fabsf(to_f32(h));
-        } else {
-          *y = static_cast<int8_t>(quant1(to_f32(h), p.out_scale));
-        }
-      }
-      if constexpr (EPI == kEpiSilu) {
-        if (p.absmax_parts != nullptr) {
-          // Row m's 8 outputs of this block sit in 8 consecutive lanes.
-#pragma unroll
-          for (int off = 1; off < 8; off <<= 1) habs = fmaxf(habs, __shfl_xor(habs, off));
-          if (c == 0 && m < p.M && nb < p.NB)
-            p.absmax_parts[static_cast<int64_t>(m) * p.NB + nb] = habs;
-        }
-      }
-    }
-  }
+  gemv_store<WAVES, MT, NBW, EPI, TY, TH>(p, red, nb0, tid, first);
 }
 
 // Batched decode, 17..64 rows with K <= 4096 (gemv_rows_kernel): a
@@ -545,6 +572,101 @@ __global__ __launch_bounds__(kRowsThreads) void gemv_rows_kernel(GemvParams p) {
   }
 }
 
+// Activations already in the packed 16x64 tiles (gemv_tiles_kernel): K > 4096
+// with few output blocks (down at 17..64 rows, and at 9..16 where the fused
+// kernels do not reach).  One workgroup of 16 wavefronts per NBW blocks, one
+// workgroup per CU; the wavefronts split K, and each streams its k-blocks of
+// the NBW weight blocks and MT activation tiles through a ring of D register
+// sets, every load one contiguous 1 KiB fragment.  The loads' ranges end at
+// the wavefront's last k-block and at the last activation tile (zeros past
+// them, no memory access), so the loop has no branch.
+//
+// Bound by the CU's memory pipeline: a workgroup reads 64 K bytes of
+// activations (M = 48: 528 KB at K = 11008) against 16 K of weights, and row-major
+// activations come 64 bytes (half a line) at a time, which costs the pipeline
+// as much as a whole line.  With gemv_kernel on row-major rows instead an MLP
+// of 4096 x 11008 at 48 rows took 52.5 us a call, of 5120 x 13824 at 16 rows
+// 62.5; with this kernel 47.0 and 53.5.
+template <int MT, int NBW>
+constexpr int tiles_depth() {  // fragments of a ring in at most 80 registers
+  return 20 / (MT + NBW) < 8 ? 20 / (MT + NBW) : 8;
+}
+
+template <int MT, int NBW, int EPI, typename TY, typename TH>
+__global__ __launch_bounds__(1024) void gemv_tiles_kernel(GemvParams p) {
+  constexpr int WAVES = 16;
+  constexpr int D = tiles_depth<MT, NBW>();
+  constexpr int TB = MT * 256;
+  __shared__ int32_t red[WAVES][NBW * TB];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int li = lane & 15;
+  const int lg = lane >> 4;
+  const int64_t nb0 = static_cast<int64_t>(blockIdx.x) * NBW;
+  const int KB = p.KB;
+  const int kb0 = KB * wave / WAVES;
+  const int nk = KB * (wave + 1) / WAVES - kb0;
+  const int MB = (p.M + 15) / 16;
+
+  FirstOutput<TY> first;
+  first.template load<MT, NBW, EPI>(p, nb0, tid);
+
+  // Blocks past the last one re-read it (their products are not stored).
+  auto rsrc = [&](const void* base, bool ok) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, ok ? nk * 1024 : 0,
+                                             kBufferWord3);
+  };
+  i32x4 wr[D][NBW], xr[D][MT];
+  auto load = [&](i32x4(&w)[NBW], i32x4(&x)[MT], int i) __attribute__((always_inline)) {
+    const int off = i * 1024 + lane * 16;
+#pragma unroll
+    for (int j = 0; j < NBW; ++j) {
+      const int64_t nb = nb0 + j < p.NB ? nb0 + j : p.NB - 1;
+      w[j] = __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                           rsrc(p.w + (nb * KB + kb0) * 64, true), off, 0, kCacheNT));
+    }
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+      x[mt] = __builtin_bit_cast(
+          i32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                     rsrc(p.xq + (static_cast<int64_t>(mt) * KB + kb0) * 1024, mt < MB), off, 0, 0));
+  };
+
+  i32x4 acc[NBW][MT];
+#pragma unroll
+  for (int j = 0; j < NBW; ++j)
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) acc[j][mt] = i32x4{0, 0, 0, 0};
+  static_for<D>([&](auto d) __attribute__((always_inline)) {
+    load(wr[decltype(d)::value], xr[decltype(d)::value], decltype(d)::value);
+  });
+  for (int i = 0; i < nk; i += D)
+    static_for<D>([&](auto d) __attribute__((always_inline)) {
+      constexpr int s = decltype(d)::value;
+#pragma unroll
+      for (int j = 0; j < NBW; ++j)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) acc[j][mt] = mfma_16x16x64(xr[s][mt], wr[s][j], acc[j][mt]);
+      load(wr[s], xr[s], i + D + s);
+    });
+
+  // C layout of v_mfma_i32_16x16x64_i8: lane (li, lg), register r holds
+  // row 4*lg + r (activation row) and column li (output within the block).
+#pragma unroll
+  for (int j = 0; j < NBW; ++j)
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        red[wave][j * TB + mt * 256 + (4 * lg + r) * 16 + li] = acc[j][mt][r];
+    }
+  __syncthreads();
+
+  gemv_store<WAVES, MT, NBW, EPI, TY, TH>(p, red, nb0, tid, first);
+}
+
 template <int MT, int CH, int RING, int EPI, typename TY, typename TH>
 hipError_t launch_rows(const GemvParams& p, hipStream_t st) {
   hipLaunchKernelGGL((gemv_rows_kernel<MT, CH, RING, EPI, TY, TH>), dim3(p.G), dim3(kRowsThreads),
@@ -562,6 +684,29 @@ hipError_t launch_rows_m(const GemvParams& p, hipStream_t st) {
     return p.NB > p.G ? launch_rows<2, 4, 3, EPI, TY, TH>(p, st)
                       : launch_rows<2, 2, 4, EPI, TY, TH>(p, st);
   return launch_rows<4, 1, 4, EPI, TY, TH>(p, st);
+}
+
+template <int NBW, int EPI, typename TY, typename TH>
+hipError_t launch_tiles_mt(const GemvParams& p, hipStream_t st) {
+  const dim3 grid(static_cast<unsigned>(ceil_div(p.NB, NBW)));
+  auto go = [&](auto mt) {
+    hipLaunchKernelGGL((gemv_tiles_kernel<decltype(mt)::value, NBW, EPI, TY, TH>), grid, dim3(1024),
+                       0, st, p);
+    return hipGetLastError();
+  };
+  if (p.M <= 16) return go(std::integral_constant<int, 1>{});
+  if (p.M <= 32) return go(std::integral_constant<int, 2>{});
+  if (p.M <= 48) return go(std::integral_constant<int, 3>{});
+  return go(std::integral_constant<int, 4>{});
+}
+
+// One block per workgroup while each CU has at most one, else two (5120
+// outputs: 160 workgroups of two rather than 256 CUs of which 64 take twice
+// the rest's work).
+template <int EPI, typename TY, typename TH>
+hipError_t launch_tiles(const GemvParams& p, hipStream_t st) {
+  return p.NB <= cu_count() ? launch_tiles_mt<1, EPI, TY, TH>(p, st)
+                            : launch_tiles_mt<2, EPI, TY, TH>(p, st);
 }
 
 template <int WAVES, int MT, int CH, int EPI, typename TY, typename TH, int NBW = 1>
@@ -610,6 +755,12 @@ bool gemv_rows_supported(int64_t M, int64_t N, int64_t K, int64_t lda, int epi) 
 
 }  // namespace
 
+bool gemv_tiles_supported(int64_t M, int64_t N, int64_t K, int epi, int y_dtype) {
+  const bool typed = epi == kEpiI32 || (epi == kEpiDequant && (y_dtype == kF16 || y_dtype == kBF16));
+  return typed && M > 8 && M <= kGemvMaxRows && K > 4096 &&
+         K < (int64_t{1} << 30) && ceil_div(N, kTileRows) <= 2 * cu_count();
+}
+
 hipError_t launch_gemv(const LinearOperands& op, hipStream_t st) {
   GemvParams p;
   p.xq = op.a;
@@ -636,6 +787,18 @@ hipError_t launch_gemv(const LinearOperands& op, hipStream_t st) {
   p.NB = static_cast<int>(nblocks);
   p.G = balanced_grid(nblocks);  // gate/up at M = 17..64: 0.3-0.5 us faster
   if (op.M <= 0 || nblocks == 0) return hipSuccess;
+  if (op.a_tiles) {
+    switch (op.epi) {
+      case kEpiI32:
+        return launch_tiles<kEpiI32, int32_t, float>(p, st);
+      case kEpiDequant:
+        if (op.y_dtype == kF16) return launch_tiles<kEpiDequant, __half, float>(p, st);
+        if (op.y_dtype == kBF16) return launch_tiles<kEpiDequant, __hip_bfloat16, float>(p, st);
+        return hipErrorInvalidValue;
+      default:
+        return hipErrorInvalidValue;
+    }
+  }
   if (fused_gemv_i8_supported(op.M, op.N, op.K, op.lda, op.epi)) return launch_gemv_fused_i8(op, st);
   if (op.res == nullptr && gemv_rows_supported(op.M, op.N, op.K, op.lda, op.epi)) {
     switch (op.epi) {

@@ -21,6 +21,7 @@ struct LinearOperands {
   // aligned, readable and zero past K up to KB*64.  GEMM: packed tiles.
   const int8_t* a;
   int64_t lda;
+  bool a_tiles = false;  // GEMV: a holds packed tiles (gemv_tiles_supported)
   const float* sx;  // per-row activation scales [M]
   const int8_t* w;  // packed weights [NB][KB] tiles
   const float* sw;  // per-output weight scales [N]
@@ -151,6 +152,11 @@ int gemm_tile_choice(int64_t MB, int64_t NB, int64_t cus);
 
 // M <= 64 (the GEMV regime).
 hipError_t launch_gemv(const LinearOperands& op, hipStream_t st);
+// Whether the GEMV takes this product's activations in the packed tiles
+// (op.a_tiles): int32 or 16-bit dequant outputs, 9..64 rows, K > 4096 and at
+// most two output blocks per CU.  Callers that write the activations
+// themselves then write tiles.
+bool gemv_tiles_supported(int64_t M, int64_t N, int64_t K, int epi, int y_dtype);
 // Any M; activations packed.
 hipError_t launch_gemm(const LinearOperands& op, hipStream_t st);
 
