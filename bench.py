@@ -465,7 +465,9 @@ def prefill_sweep(layers, device, m: int = 560) -> dict:
             row[f"{key}_TOPS"] = round(ops / (per * 1e-3) / 1e12, 1)
         row["gemm_kernel_frac_int8_peak"] = round(
             ops / (timed["gemm_kernel"] * 1e-3) / 1e12 / INT8_PEAK_TOPS, 4)
-        row["tile"] = names[lib.w8a8_gemm_tile_config(m, spec.n, cus)]
+        pipe = lib.w8a8_gemm_pipe_config(m, spec.n, spec.k, cus)
+        row["tile"] = (f"pipe-{_lib.GEMM_PIPE_NAMES[pipe]}" if pipe >= 0 else
+                       names[lib.w8a8_gemm_tile_config(m, spec.n, cus)])
         out[spec.name] = row
     torch.cuda.synchronize()
     return out

@@ -109,9 +109,17 @@ int64_t w8a8_packed_bytes(int64_t rows, int64_t k);
  * for an [m, k] activation. */
 int64_t w8a8_workspace_bytes(int64_t m, int64_t k);
 
+/* Pipelined GEMM tile (8 wavefronts, one workgroup per CU) for an m x n x k
+ * product in the GEMM regime on a device with `cus` compute units: 0 =
+ * 128x128, 1 = 192x160, 2 = 256x128, 3 = 256x192, 4 = 192x288, 5 = 256x256,
+ * 6 = 256x352; -1 where none is taken (K below 1024, at most 64 rows, too few
+ * tiles for the CUs, or a size not positive) and the tile of
+ * w8a8_gemm_tile_config is.  A pure function of its arguments. */
+int w8a8_gemm_pipe_config(int64_t m, int64_t n, int64_t k, int64_t cus);
+
 /* GEMM workgroup tile that w8a8_gemm_i32 / w8a8_linear / w8a8_linear_i8in
- * launch for an m x n product in the GEMM regime, on a device with `cus`
- * compute units: 0 = 32x32 (one wave, ring stages of four k-blocks), 1 =
+ * launch for an m x n product in the GEMM regime that takes no pipelined tile
+ * (w8a8_gemm_pipe_config), on a device with `cus` compute units: 0 = 32x32 (one wave, ring stages of four k-blocks), 1 =
  * 64x64 (stages of four k-blocks), 2 = 128x128 (one workgroup per CU, stages
  * of two k-blocks), 3 = 128x128, 4 = 128x192, 5 = 128x224, 6 = 128x256,
  * 7 = 256x256 (one workgroup per CU, stages of two k-blocks), 8 = 64x32

@@ -485,6 +485,12 @@ int w8a8_gemm_tile_config(int64_t m, int64_t n, int64_t cus) {
   return gemm_tile_choice(ceil_div(m, kTileRows), ceil_div(n, kTileRows), cus);
 }
 
+int w8a8_gemm_pipe_config(int64_t m, int64_t n, int64_t k, int64_t cus) {
+  if (m <= 0 || n <= 0 || k <= 0 || cus <= 0 || m > kMaxRows || n > kMaxRows || k > kMaxRows)
+    return kPipeNone;
+  return gemm_pipe_choice(ceil_div(m, kTileRows), ceil_div(n, kTileRows), ceil_div(k, kTileK), cus);
+}
+
 int w8a8_quant_rows(const void* x, int x_dtype, int64_t rows, int64_t k, int64_t ldx,
                     int8_t* q, int64_t ldq, float* scales, hipStream_t stream) {
   if (rows < 0 || k < 0 || rows > kMaxRows) return W8A8_ERR_SHAPE;

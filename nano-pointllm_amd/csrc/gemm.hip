@@ -475,10 +475,11 @@ __device__ inline __amdgpu_buffer_rsrc_t dma_rsrc(const void* base) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, 0x7fffffff, 0x00020000);
 }
 
-// 16 bytes per lane from the buffer at voffset into LDS at lds + 16 * lane
-// (buffer_load_dwordx4 ... lds).
-__device__ inline void dma16(__amdgpu_buffer_rsrc_t r, void* lds, uint32_t voffset) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void*)lds, 16, voffset, 0, 0, 0);
+// 16 bytes per lane from the buffer at voffset + soffset (wave-uniform) into
+// LDS at lds + 16 * lane (buffer_load_dwordx4 ... lds).
+__device__ inline void dma16(__amdgpu_buffer_rsrc_t r, void* lds, uint32_t voffset,
+                             uint32_t soffset = 0) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void*)lds, 16, voffset, soffset, 0, 0);
 }
 
 // Weights-direct GEMM: NW wavefronts, each owning all A 16-row activation
@@ -615,6 +616,145 @@ __global__ __launch_bounds__(NW * 64, NW / 4) void gemm_wd_kernel(GemmParams p) 
   store_tile<1, NW, A, B, kLds, EPI, TY, TH>(p, acc, 0, wave, mb0, nb0, lane, lds, scales);
 }
 
+// Pipelined GEMM: WM x WN = 8 wavefronts, one workgroup per CU, each wavefront
+// BR x BC 16x16 blocks (tile 16 WM BR x 16 WN BC), an S-slot LDS ring of single
+// k-blocks (64 K) and one barrier per k-block.
+//   * Each wavefront keeps the fragments of its shorter side of a k-block in
+//     registers (`held`, double-buffered) and passes the longer side's through
+//     R registers (`strm`), every fragment read from LDS about a k-block before
+//     its MFMAs, also across the barriers: no MFMA waits for an LDS read
+//     issued behind a barrier.  (gemm_kernel reads a k-block's fragments after
+//     its barrier, so all wavefronts read at once while the matrix pipes idle.)
+//   * The k-loop has no branch: operand copies past the last k-block re-read it
+//     into slots that nothing reads, and wavefronts without a share of their
+//     own copy the last fragment again (the same bytes to the same place), so
+//     every wait is a fixed count and the compiler schedules whole k-blocks.
+//   * Copies are LDS-DMA buffer loads with the k-block as scalar offset, issued
+//     between the MFMAs.
+// What bounds it: the k-loop runs at 1.62 thousand shader cycles a k-block on
+// 256 x 352 (1.41 of them MFMA), 1.27 (1.02) on 256 x 256, 0.50 (0.26) on
+// 128 x 128, where the operands, cold and shared by a few CUs, arrive at 55 to 70
+// GB/s per CU; with every CU busy the shader clock falls from 2.4 to 1.7-2.0 GHz
+// (power: with zero operands it stays at 2.4).  Two k-blocks per barrier, deeper
+// rings and other orders of the LDS reads all measured the same or slower.
+template <int WM, int WN, int BR, int BC, int S, int R, int EPI, typename TY, typename TH>
+__global__ __launch_bounds__(WM * WN * 64, WM * WN / 4) void gemm_pipe_kernel(GemmParams p) {
+  constexpr int NW = WM * WN;
+  constexpr int BMF = WM * BR;             // 16-row activation tiles per k-block
+  constexpr int BNF = WN * BC;             // 16-row weight tiles per k-block
+  constexpr int F = BMF + BNF;
+  constexpr int LPW = (F + NW - 1) / NW;   // fragment copies per wavefront and k-block
+  constexpr bool kHoldB = BC <= BR;
+  constexpr int NH = kHoldB ? BC : BR;     // held fragments
+  constexpr int NS = kHoldB ? BR : BC;     // streamed fragments
+  // At k-block kb's barrier kb and kb + 1 are in the ring, kb - 1's slot is
+  // free, and the S - 3 slots between are being filled.
+  static_assert(S >= 3 && NW % 4 == 0 && R <= NS && LPW <= NS, "ring shape");
+  using Scales = TileScales<EPI, 16 * BMF, 16 * BNF>;
+  constexpr int kRing = S * F * 1024;
+  __shared__ i32x4 smem[(kRing + sizeof(Scales)) / 16];  // one array, as in gemm_kernel
+  auto lds = reinterpret_cast<i32x4 (*)[F][64]>(smem);
+  Scales& scales = *reinterpret_cast<Scales*>(smem + kRing / 16);
+
+  const int b = blockIdx.x;
+  const int tile = (b % kXcds) * p.per_xcd + b / kXcds;
+  if (tile >= p.tiles) return;
+  const int mb0 = (tile % p.tiles_m) * BMF;
+  const int nb0 = (tile / p.tiles_m) * BNF;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave / WN;
+  const int wn = wave % WN;
+  const int KB = p.KB;
+
+  // Fragment g < BMF of a k-block is activation block mb0 + g, the others
+  // weight block nb0 + g - BMF, clamped to the operand's last block (products
+  // that the epilogue never stores).
+  const i32x4* src[LPW];
+  int frag[LPW];
+#pragma unroll
+  for (int q = 0; q < LPW; ++q) {
+    const int g = min(q * NW + wave, F - 1);
+    frag[q] = g;
+    src[q] = g < BMF ? p.a + static_cast<int64_t>(min(mb0 + g, p.MB - 1)) * KB * 64
+                     : p.w + static_cast<int64_t>(min(nb0 + g - BMF, p.NB - 1)) * KB * 64;
+  }
+  auto copy = [&](int kb, int slot, int q) __attribute__((always_inline)) {
+    dma16(dma_rsrc(src[q]), &lds[slot][frag[q]][0], lane * 16, kb * 1024);
+  };
+
+  i32x4 acc[BR][BC];
+#pragma unroll
+  for (int i = 0; i < BR; ++i)
+#pragma unroll
+    for (int j = 0; j < BC; ++j) acc[i][j] = i32x4{0, 0, 0, 0};
+
+  scales.template load<NW>(p, mb0, nb0, wave, lane);
+#pragma unroll
+  for (int s = 0; s < S - 1; ++s)
+#pragma unroll
+    for (int q = 0; q < LPW; ++q) copy(min(s, KB - 1), s, q);
+  wait_vmcnt<LPW * (S - 2)>();  // k-block 0
+  ring_barrier_tracked();
+  const int hoff = kHoldB ? BMF + wn * BC : wm * BR;
+  const int soff = kHoldB ? wm * BR : BMF + wn * BC;
+  i32x4 held[2][NH], strm[R];
+#pragma unroll
+  for (int j = 0; j < NH; ++j) held[0][j] = lds[0][hoff + j][lane];
+#pragma unroll
+  for (int i = 0; i < R; ++i) strm[i] = lds[0][soff + i][lane];
+
+  int slot = 0;       // of k-block kb
+  int fill = S - 1;   // of k-block kb + S - 1
+  // k-block kb, the I-th of an unrolled group: streamed fragment i sits in
+  // register (I NS + i) % R, the held ones in set I % 2.
+  auto step = [&](int kb, auto idx) __attribute__((always_inline)) {
+    constexpr int I = decltype(idx)::value;
+    constexpr int cur = I % 2;
+    const int next = slot + 1 == S ? 0 : slot + 1;
+    const int fkb = min(kb + S - 1, KB - 1);
+    // k-block kb + 1 has landed, and every wavefront has read kb - 1 (its
+    // MFMAs, issued above, waited for the reads), whose slot is refilled.
+    wait_vmcnt<LPW * (S - 3)>();
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    static_for<NS>([&](auto ic) __attribute__((always_inline)) {
+      constexpr int i = decltype(ic)::value;
+      constexpr int reg = (I * NS + i) % R;
+#pragma unroll
+      for (int q = i * LPW / NS; q < (i + 1) * LPW / NS; ++q) copy(fkb, fill, q);
+#pragma unroll
+      for (int j = 0; j < NH; ++j) {
+        if constexpr (kHoldB) {
+          acc[i][j] = mfma_16x16x64(held[cur][j], strm[reg], acc[i][j]);
+        } else {
+          acc[j][i] = mfma_16x16x64(strm[reg], held[cur][j], acc[j][i]);
+        }
+      }
+      // The fragment R ahead takes the register just used; past the last
+      // k-block these reads bring stale bytes that no MFMA takes.
+      strm[reg] = i + R < NS ? lds[slot][soff + i + R][lane] : lds[next][soff + i + R - NS][lane];
+#pragma unroll
+      for (int j = i * NH / NS; j < (i + 1) * NH / NS; ++j)
+        held[cur ^ 1][j] = lds[next][hoff + j][lane];
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    slot = next;
+    fill = fill + 1 == S ? 0 : fill + 1;
+  };
+  // Unrolled until the register sets repeat.
+  constexpr int U = (2 * NS) % R == 0 ? 2 : 2 * R;
+  int kb = 0;
+  for (; kb + U <= KB; kb += U)
+    static_for<U>([&](auto i) __attribute__((always_inline)) { step(kb + decltype(i)::value, i); });
+  static_for<U>([&](auto i) __attribute__((always_inline)) {
+    if (kb + decltype(i)::value < KB) step(kb + decltype(i)::value, i);
+  });
+
+  wait_vmcnt<0>();  // copies past the last k-block, before the epilogue reuses the ring
+  store_tile<WM, WN, BR, BC, kRing, EPI, TY, TH>(p, acc, wm, wn, mb0, nb0, lane, smem, scales);
+}
+
 // Launches the weights-direct kernel for the problem in p.
 template <int NW, int A, int B, int D, int EPI, typename TY, typename TH>
 hipError_t launch_wd(GemmParams p, hipStream_t st) {
@@ -627,6 +767,20 @@ hipError_t launch_wd(GemmParams p, hipStream_t st) {
   p.per_xcd = static_cast<int>(ceil_div(tiles, kXcds));
   hipLaunchKernelGGL((gemm_wd_kernel<NW, A, B, D, EPI, TY, TH>), dim3(p.per_xcd * kXcds),
                      dim3(NW * 64), 0, st, p);
+  return hipGetLastError();
+}
+
+// Launches a pipelined tile for the problem in p.
+template <int WM, int WN, int BR, int BC, int S, int R, int EPI, typename TY, typename TH>
+hipError_t launch_pipe(GemmParams p, hipStream_t st) {
+  const int64_t tiles_m = ceil_div(p.MB, WM * BR);
+  const int64_t tiles = tiles_m * ceil_div(p.NB, WN * BC);
+  if (ceil_div(tiles, kXcds) * kXcds > INT32_MAX) return hipErrorInvalidConfiguration;
+  p.tiles_m = static_cast<int>(tiles_m);
+  p.tiles = static_cast<int>(tiles);
+  p.per_xcd = static_cast<int>(ceil_div(tiles, kXcds));
+  hipLaunchKernelGGL((gemm_pipe_kernel<WM, WN, BR, BC, S, R, EPI, TY, TH>),
+                     dim3(p.per_xcd * kXcds), dim3(WM * WN * 64), 0, st, p);
   return hipGetLastError();
 }
 
@@ -686,6 +840,24 @@ hipError_t launch_cfg(GemmParams p, hipStream_t st) {
 //     it gains nothing.
 template <int EPI, typename TY, typename TH>
 hipError_t launch_t(const GemmParams& p, hipStream_t st) {
+  switch (gemm_pipe_choice(p.MB, p.NB, p.KB, cu_count())) {
+    case kPipe256x352:
+      return launch_pipe<4, 2, 4, 11, 4, 3, EPI, TY, TH>(p, st);
+    case kPipe256x256:
+      return launch_pipe<4, 2, 4, 8, 4, 4, EPI, TY, TH>(p, st);
+    case kPipe256x192:
+      return launch_pipe<4, 2, 4, 6, 5, 6, EPI, TY, TH>(p, st);
+    case kPipe256x128:
+      return launch_pipe<4, 2, 4, 4, 6, 4, EPI, TY, TH>(p, st);
+    case kPipe192x288:
+      return launch_pipe<4, 2, 3, 9, 5, 3, EPI, TY, TH>(p, st);
+    case kPipe192x160:
+      return launch_pipe<4, 2, 3, 5, 7, 5, EPI, TY, TH>(p, st);
+    case kPipe128x128:
+      return launch_pipe<2, 4, 4, 2, 9, 4, EPI, TY, TH>(p, st);
+    default:
+      break;
+  }
   switch (gemm_tile_choice(p.MB, p.NB, cu_count())) {
     case kGemmTinyDeep:
       return launch_cfg<1, 1, 2, 2, 3, 4, 4, EPI, TY, TH>(p, st);
@@ -715,6 +887,43 @@ hipError_t launch_t(const GemmParams& p, hipStream_t st) {
 }
 
 }  // namespace
+
+// The pipelined tile whose rounds over the CUs take least, by the time of one
+// of its k-steps with all CUs busy (nanoseconds, measured at K = 4096 and
+// 11008: the wider the tile, the less per product).  So packed QKV takes
+// 192x160 at 560 rows (231 tiles, 33.4 us; 35.2 on the weights-direct tile)
+// and 256x192 at 2048 (two full rounds, 91 us against 104 for 128x256), gate/up
+// 192x288 at 560 (52.7 against 63.9 for 128x224) and 256x352 at 1024 and 2048
+// (82 against 105, 153 against 179), O and down 128x128 at 560 (18.6 / 41.5
+// against 20.4 / 49 for 112x96) and 1024 (51 against 57 for the ring of 16
+// wavefronts) and 256x128 at 2048 (34 / 77 against 38 / 99).
+// Taken where the tiles fill three fifths of the CUs; below that the smaller
+// ring tiles cover more of them, and below 16 k-blocks filling the ring (up to
+// 8) would be a large part of the work.
+int gemm_pipe_choice(int64_t MB, int64_t NB, int64_t KB, int64_t cus) {
+  struct Tile {
+    GemmPipe id;
+    int mb, nb, step_ns;
+  };
+  static constexpr Tile kTiles[] = {
+      {kPipe256x352, 16, 22, 880}, {kPipe256x256, 16, 16, 670}, {kPipe192x288, 12, 18, 600},
+      {kPipe256x192, 16, 12, 560}, {kPipe256x128, 16, 8, 435},  {kPipe192x160, 12, 10, 400},
+      {kPipe128x128, 8, 8, 275},
+  };
+  if (MB <= 4 || KB < 16 || KB >= (int64_t{1} << 20)) return kPipeNone;
+  int best = kPipeNone;
+  int64_t best_ns = 0, best_tiles = 0;
+  for (const Tile& t : kTiles) {
+    const int64_t tiles = ceil_div(MB, t.mb) * ceil_div(NB, t.nb);
+    const int64_t ns = ceil_div(tiles, cus) * t.step_ns;
+    if (best == kPipeNone || ns < best_ns) {
+      best = t.id;
+      best_ns = ns;
+      best_tiles = tiles;
+    }
+  }
+  return 5 * best_tiles >= 3 * cus ? best : kPipeNone;
+}
 
 int gemm_tile_choice(int64_t MB, int64_t NB, int64_t cus) {
   // The 112 x 256 weights-direct tile when one round of it (one workgroup per

@@ -150,6 +150,21 @@ enum GemmTile : int {
 };
 int gemm_tile_choice(int64_t MB, int64_t NB, int64_t cus);
 
+// Pipelined GEMM tiles (gemm_pipe_kernel, 8 wavefronts, one workgroup per CU),
+// taken before the ring tiles above: gemm_pipe_choice's answer for MB x NB
+// blocks over KB k-blocks (64 K), or kPipeNone.
+enum GemmPipe : int {
+  kPipeNone = -1,
+  kPipe128x128 = 0,
+  kPipe192x160 = 1,
+  kPipe256x128 = 2,
+  kPipe256x192 = 3,
+  kPipe192x288 = 4,
+  kPipe256x256 = 5,
+  kPipe256x352 = 6,
+};
+int gemm_pipe_choice(int64_t MB, int64_t NB, int64_t KB, int64_t cus);
+
 // M <= 64 (the GEMV regime).
 hipError_t launch_gemv(const LinearOperands& op, hipStream_t st);
 // Whether the GEMV takes this product's activations in the packed tiles

@@ -29,6 +29,8 @@ NOALLOC_SCRATCH_BYTES = 16 << 20
 # Names of the GEMM tiles w8a8_gemm_tile_config returns, by code.
 GEMM_TILE_NAMES = ("tiny-deep", "small-deep", "big-deep", "big", "w192", "w224", "w256",
                    "w256sq", "mid", "wd7x2", "t112x96", "t128x96")
+# Names of the pipelined GEMM tiles w8a8_gemm_pipe_config returns, by code.
+GEMM_PIPE_NAMES = ("128x128", "192x160", "256x128", "256x192", "192x288", "256x256", "256x352")
 
 _TORCH_TO_CODE = {
     torch.float32: F32,
@@ -45,6 +47,7 @@ EXPORTED_SYMBOLS = (
     "w8a8_packed_bytes",
     "w8a8_workspace_bytes",
     "w8a8_gemm_tile_config",
+    "w8a8_gemm_pipe_config",
     "w8a8_quant_rows",
     "w8a8_qdq_rows",
     "w8a8_quant_rows_scaled",
@@ -83,6 +86,7 @@ _SIGNATURES = {
     "w8a8_packed_bytes": (_i64, [_i64, _i64]),
     "w8a8_workspace_bytes": (_i64, [_i64, _i64]),
     "w8a8_gemm_tile_config": (_int, [_i64, _i64, _i64]),
+    "w8a8_gemm_pipe_config": (_int, [_i64, _i64, _i64, _i64]),
     "w8a8_quant_rows": (_int, [_vp, _int, _i64, _i64, _i64, _vp, _i64, _vp, _vp]),
     "w8a8_qdq_rows": (_int, [_vp, _int, _i64, _i64, _i64, _i64, _vp, _i64, _vp, _i64, _vp, _vp]),
     "w8a8_quant_rows_scaled": (_int, [_vp, _int, _i64, _i64, _i64, _vp, _i64, _vp, _i64, _vp]),
