@@ -126,7 +126,7 @@ __device__ inline void prologue_vec(const PrologueParams& p, float* red) {
   constexpr bool kHalf = std::is_same<TX, __half>::value;
   constexpr bool kW16 = sizeof(TW) == 2;
   auto as_h2 = [](uint32_t u) { return __builtin_bit_cast(h2, u); };
-  const int64_t row = blockIdx.x;
+  const int64_t row = p.KB > 0 ? packed_row_of(blockIdx.x, gridDim.x) : blockIdx.x;
   const int tid = threadIdx.x;
   const int K = static_cast<int>(p.K);
   const __amdgpu_buffer_rsrc_t xd =
@@ -279,7 +279,7 @@ template <typename TX, typename TW, int REG, bool VEC>
 __global__ __launch_bounds__(kProThreads) void prologue_quant_kernel(PrologueParams p) {
   using TY = TW;
   __shared__ float red[kProThreads / 8];
-  const int64_t row = blockIdx.x;
+  const int64_t row = p.KB > 0 ? packed_row_of(blockIdx.x, gridDim.x) : blockIdx.x;
   const int tid = threadIdx.x;
   const int64_t K = p.K;
   if (p.KB > 0 && row >= p.M) {

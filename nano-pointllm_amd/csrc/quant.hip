@@ -92,7 +92,7 @@ __global__ __launch_bounds__(NT) void quant_rows_kernel(
     const float* __restrict__ scale_in, int64_t scale_stride, int8_t* __restrict__ q,
     int64_t ldq, int64_t ncols_out, int vec_out, int64_t KB, float* __restrict__ scales_out) {
   __shared__ float red[NT / 64];
-  const int64_t row = blockIdx.x;
+  const int64_t row = PACKED ? packed_row_of(blockIdx.x, gridDim.x) : blockIdx.x;
   const int tid = threadIdx.x;
   const bool live = row < rows;
   const TX* xr = x + (live ? row : 0) * ldx;

@@ -225,8 +225,7 @@ __device__ inline float mul_keep_sign(float a, float b) {
 // largest one is normal), one Newton correction of the quotient, and
 // v_div_fixup_f32 for infinities and NaN.  14 instructions where expf and the
 // IEEE division take about 30: the SiLU epilogue of a 256 x 256 GEMM tile is
-// bound by them (together with the pipelined tiles it took 2048 x 22016 x 4096
-// from 179 to 146 us).
+// bound by them (2048 x 22016 x 4096 on the pipelined tiles: 153 -> 143 us).
 __device__ inline float silu_f32(float g) {
   // Past +-128 the quotient no longer depends on exp (2^185 overflows to
   // infinity, 2^-185 vanishes against 1).
@@ -435,6 +434,17 @@ __device__ inline float tree8_sum(float v) {
 __device__ inline float tree8_sum_lane(const float (&s)[8]) {
   return __fadd_rn(__fadd_rn(__fadd_rn(s[0], s[1]), __fadd_rn(s[2], s[3])),
                    __fadd_rn(__fadd_rn(s[4], s[5]), __fadd_rn(s[6], s[7])));
+}
+
+// Row of workgroup `block` of `blocks`, one workgroup per row, where the rows
+// go to packed tiles.  The eight rows 8i .. 8i+7 share every 128-byte line of a
+// tile, and workgroup b runs on XCD b % 8: taken in order they would write each
+// line from eight L2 caches, 16 bytes each.  Every whole group of 64 workgroups
+// is transposed, so that eight such rows meet in one L2 (the rest in order).
+// 2048 x 11008 binary16: 24.5 -> 16.8 us, 560 x 11008 9.1 -> 7.7, 560 x 4096
+// 5.8 -> 4.5, the RMSNorm prologue at 560 x 4096 8.9 -> 6.4.
+__device__ inline int64_t packed_row_of(uint32_t block, uint32_t blocks) {
+  return (block | 63u) < blocks ? (block & ~63u) + ((block & 7u) << 3) + ((block >> 3) & 7u) : block;
 }
 
 // Packed-tile byte offset of element (r, k) of a [rows, K] operand.
