@@ -180,12 +180,13 @@ inline bool use_gemv(int64_t m, int64_t n, int64_t k) {
 }
 
 // Runs the int8 product for activations already staged in `act` (row-major
-// [m, round_up(k,64)] for the GEMV, packed tiles for the GEMM).  The GEMV
-// kernels take the residual-add epilogue (op.res) themselves; the GEMM
-// writes its output first and the add runs over it.
+// [m, round_up(k,64)] for the GEMV, packed tiles for the GEMM).  The kernels
+// take the residual-add epilogue (op.res) themselves; only where its RMSNorm
+// chunk sums are wanted too the GEMM writes its output first and the add runs
+// over it.
 inline hipError_t run_product(const LinearOperands& op, hipStream_t st) {
   if (op.a_tiles || use_gemv(op.M, op.N, op.K)) return launch_gemv(op, st);
-  if (op.res == nullptr) return launch_gemm(op, st);
+  if (op.ss_parts == nullptr) return launch_gemm(op, st);
   LinearOperands plain = op;
   plain.res = nullptr;
   plain.ss_parts = nullptr;

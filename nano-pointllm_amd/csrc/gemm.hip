@@ -50,6 +50,9 @@ struct GemmParams {
   const int32_t* rq_shift;
   const int32_t* rq_bias;
   float* absmax_parts;  // kEpiSilu: [M][NB] per-block row |h|max (nullable)
+  // kEpiDequant with 16-bit outputs (nullable): the residual rows added to them.
+  const void* res;
+  int64_t ld_res;
   int M;
   int N;
   int MB;
@@ -163,7 +166,9 @@ struct TileScales {
 // With a row per register instead (a row scale per accumulator, each loaded
 // from memory behind a bounds check, and 2-byte LDS writes) these took 32,
 // 16.6 and 47.  A 2048 x 22016 x 4096 SiLU product went from 191 to 177 us.
-template <int WM, int WN, int BR, int BC, int STAGE_BYTES, int EPI, typename TY, typename TH>
+// ROOMY: the kernel has registers for residual chunks beside its accumulators.
+template <int WM, int WN, int BR, int BC, int STAGE_BYTES, int EPI, typename TY, typename TH,
+          bool ROOMY = false>
 __device__ inline void store_tile(const GemmParams& p, i32x4 (&acc)[BR][BC], int wm, int wn,
                                   int mb0, int nb0, int lane, void* stage,
                                   const TileScales<EPI, 16 * WM * BR, 16 * WN * BC>& ts) {
@@ -282,9 +287,37 @@ __device__ inline void store_tile(const GemmParams& p, i32x4 (&acc)[BR][BC], int
     const int64_t n0_out = kHalfCols ? n0 / 2 : n0;
     const int crow = static_cast<int>(threadIdx.x) / CPR;
     const int cchunk = static_cast<int>(threadIdx.x) % CPR;
+    const int64_t nc = n0_out + cchunk * EV;  // this thread's first output column
+    // Output row of tile-local row `row` of the pass over blocks i0 .. i0 + ni.
+    auto out_row = [&](int row, int i0, int ni) {
+      return m0 + 16 * (row / (16 * ni) * BR + i0) + row % (16 * ni);
+    };
+    // Residual add, y = dtype(dtype(dequant) + res); with ROOMY the pass's
+    // residual chunks (up to 8 per thread) are requested before its arithmetic.
+    // It spares O and down of a prefill layer a pass over their rows (three
+    // trips through memory).
+    constexpr bool kRes = EPI == kEpiDequant && kOutBytes == 2;
+    constexpr int kSweeps = (WM * 16 * IPP + RPP - 1) / RPP;
+    constexpr bool kEarly = kRes && ROOMY && kSweeps <= 8;
+    const bool res_vec = kRes && p.res != nullptr && nc + EV <= n_out_total &&
+                         ((reinterpret_cast<uintptr_t>(p.res) |
+                           static_cast<uintptr_t>(p.ld_res * kOutBytes)) & 15) == 0;
+    [[maybe_unused]] Pack<TY, EV> early[kEarly ? kSweeps : 1];
 #pragma unroll
     for (int i0 = 0; i0 < BR; i0 += IPP) {
       const int ni = BR - i0 < IPP ? BR - i0 : IPP;  // compile-time after unrolling
+      if constexpr (kEarly) {
+        if (res_vec) {
+#pragma unroll
+          for (int t = 0; t < kSweeps; ++t) {
+            const int row = t * RPP + crow;
+            const int64_t m = out_row(row, i0, ni);
+            const bool ok = crow < RPP && row < WM * 16 * ni && m < p.M;
+            early[t] = *reinterpret_cast<const Pack<TY, EV>*>(
+                static_cast<const TY*>(p.res) + (ok ? m : 0) * p.ld_res + nc);
+          }
+        }
+      }
       ring_barrier();  // the ring's (or the last pass's) readers are done
 #pragma unroll
       for (int j = 0; j < BC; ++j) {
@@ -314,11 +347,32 @@ __device__ inline void store_tile(const GemmParams& p, i32x4 (&acc)[BR][BC], int
 #pragma unroll
       for (int base = 0; base < rows; base += RPP) {
         const int row = base + crow;
-        const int64_t m = m0 + 16 * (row / (16 * ni) * BR + i0) + row % (16 * ni);
-        const int64_t n = n0_out + cchunk * EV;
+        const int64_t m = out_row(row, i0, ni);
+        const int64_t n = nc;
         if (crow < RPP && row < rows && m < p.M && n < n_out_total) {
           TY* const dst = static_cast<TY*>(p.y) + m * p.ldy + n;
-          const TY* const src = reinterpret_cast<const TY*>(st + row * kStride + cchunk * 16);
+          Pack<TY, EV>& out = *reinterpret_cast<Pack<TY, EV>*>(st + row * kStride + cchunk * 16);
+          if constexpr (kRes) {
+            if (p.res != nullptr) {
+              const TY* const r = static_cast<const TY*>(p.res) + m * p.ld_res + n;
+              Pack<TY, EV> o = out;
+              if (res_vec) {
+                Pack<TY, EV> a;
+                if constexpr (kEarly) {
+                  a = early[base / RPP];
+                } else {
+                  a = *reinterpret_cast<const Pack<TY, EV>*>(r);
+                }
+#pragma unroll
+                for (int e = 0; e < EV; ++e) o.v[e] = add_rounded(o.v[e], a.v[e]);
+              } else {
+                for (int e = 0; e < EV; ++e)
+                  if (n + e < n_out_total) o.v[e] = add_rounded(o.v[e], r[e]);
+              }
+              out = o;
+            }
+          }
+          const TY* const src = out.v;
           if (vec_ok && n + EV <= n_out_total) {
             *reinterpret_cast<i32x4*>(dst) = *reinterpret_cast<const i32x4*>(src);
           } else {
@@ -752,7 +806,7 @@ __global__ __launch_bounds__(WM * WN * 64, WM * WN / 4) void gemm_pipe_kernel(Ge
   });
 
   wait_vmcnt<0>();  // copies past the last k-block, before the epilogue reuses the ring
-  store_tile<WM, WN, BR, BC, kRing, EPI, TY, TH>(p, acc, wm, wn, mb0, nb0, lane, smem, scales);
+  store_tile<WM, WN, BR, BC, kRing, EPI, TY, TH, true>(p, acc, wm, wn, mb0, nb0, lane, smem, scales);
 }
 
 // Launches the weights-direct kernel for the problem in p.
@@ -989,6 +1043,8 @@ hipError_t launch_gemm(const LinearOperands& op, hipStream_t st) {
   p.rq_shift = op.rq_shift;
   p.rq_bias = op.rq_bias;
   p.absmax_parts = op.absmax_parts;
+  p.res = op.res;
+  p.ld_res = op.ld_res;
   p.M = static_cast<int>(op.M);
   p.N = static_cast<int>(op.N);
   p.MB = static_cast<int>(ceil_div(op.M, kTileRows));

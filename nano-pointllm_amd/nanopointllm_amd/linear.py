@@ -200,7 +200,8 @@ class W8A8Linear(nn.Module):
         return _w.linear_i8in(xq, x_scale, p.packed, p.scale, p.bias, p.out_features,
                               out_dtype=out_dtype, in_features=p.in_features)
 
-    def forward_residual(self, x: torch.Tensor, residual: torch.Tensor) -> _w.ResidualOutput:
+    def forward_residual(self, x: torch.Tensor, residual: torch.Tensor, *,
+                         ss_parts: bool = True) -> _w.ResidualOutput:
         """``residual + self(x)`` in the activation dtype with the RMSNorm
         chunk sums of the result (``linear_residual``): the residual add of a
         decoder layer after o_proj / down_proj (lightweight_runner.py:247-257,
@@ -209,14 +210,15 @@ class W8A8Linear(nn.Module):
             raise ValueError("the residual-add epilogue takes per-token dynamic activations")
         p = self.weight_q
         return _w.linear_residual(x, p.packed, p.scale, p.bias, p.out_features, residual,
-                                  in_features=p.in_features)
+                                  ss_parts=ss_parts, in_features=p.in_features)
 
     def forward_i8_residual(self, xq: torch.Tensor, x_scale: torch.Tensor,
-                            residual: torch.Tensor) -> _w.ResidualOutput:
+                            residual: torch.Tensor, *, ss_parts: bool = True
+                            ) -> _w.ResidualOutput:
         """:meth:`forward_residual` on int8 activations with per-row scales."""
         p = self.weight_q
         return _w.linear_i8in_residual(xq, x_scale, p.packed, p.scale, p.bias, p.out_features,
-                                       residual, in_features=p.in_features)
+                                       residual, ss_parts=ss_parts, in_features=p.in_features)
 
     def accumulators(self, x: torch.Tensor) -> torch.Tensor:
         """Raw int32 accumulators of ``forward`` (for exactness checks)."""
@@ -459,14 +461,16 @@ class W8A8MLP(nn.Module):
         return first.residual, self.down.forward_i8(first.y, self._h_rows(first.y),
                                                     out_dtype=hidden_states.dtype)
 
-    def forward_rmsnorm_ss_residual(self, hidden_states: torch.Tensor, ss_parts: torch.Tensor,
-                                    norm: nn.Module) -> _w.ResidualOutput:
+    def forward_rmsnorm_ss_residual(self, hidden_states: torch.Tensor,
+                                    ss_parts: torch.Tensor | None, norm: nn.Module
+                                    ) -> _w.ResidualOutput:
         """``hidden_states + mlp(norm(hidden_states))`` for rows that a
         residual-add linear wrote with their RMSNorm chunk sums ``ss_parts``
         (the o_proj of :meth:`W8A8Linear.forward_residual`): the norm and
         gate/up run as one launch that reads the sums, and down adds the
         rows back in its epilogue and returns the next norm's sums
-        (lightweight_runner.py:247-257, 320-383, 552)."""
+        (lightweight_runner.py:247-257, 320-383, 552).  With ``ss_parts`` None
+        the norm sums the rows itself and no sums come back."""
         p = self.gate_up.weight_q
         epi = _lib.EPI_SILU_MUL if self.h_scale is None else _lib.EPI_SILU_MUL_Q8
         h = _w.rmsnorm_linear(hidden_states, norm.weight, _norm_eps(norm), p.packed, p.scale,
@@ -474,8 +478,9 @@ class W8A8MLP(nn.Module):
                               y_scale=0.0 if self.h_scale is None else self.h_scale,
                               in_features=p.in_features, ss_parts=ss_parts).y
         if self.h_scale is None:
-            return self.down.forward_residual(h, hidden_states)
-        return self.down.forward_i8_residual(h, self._h_rows(h), hidden_states)
+            return self.down.forward_residual(h, hidden_states, ss_parts=ss_parts is not None)
+        return self.down.forward_i8_residual(h, self._h_rows(h), hidden_states,
+                                             ss_parts=ss_parts is not None)
 
     def forward_i8(self, xq: torch.Tensor, x_scale: torch.Tensor, *,
                    out_dtype: torch.dtype = torch.float16) -> torch.Tensor:

@@ -58,6 +58,9 @@ from .inject import inject_w8a8
 from .lm_head import DecodeLMHead
 from .linear import W8A8Linear, W8A8MLP, W8A8PackedQKV, _norm_eps
 
+#: Most rows the GEMV kernels take (kGemvMaxRows).
+GEMV_MAX_ROWS = 64
+
 AttentionCore = Callable[[torch.Tensor, torch.Tensor, torch.Tensor, int, Any], torch.Tensor]
 
 
@@ -97,6 +100,24 @@ class W8A8LlamaLayer(nn.Module):
         self.mlp = w8a8_mlp
         self.attention_core = attention_core
 
+    def _adds_in_epilogues(self, context: torch.Tensor, rows: torch.Tensor) -> bool:
+        """Whether both residual adds go into the epilogues of o_proj and down:
+        past the GEMV's rows, where the GEMM adds them as it writes (at fewer
+        rows the plain kernels are the faster ones), for 16-bit rows of one
+        dtype, per-token o_proj activations, and modules whose calls nothing
+        observes (the epilogue route goes past ``__call__`` and its hooks).
+        The bits are the same: one rounding of the sum either way."""
+        o, down = self.o_proj, self.mlp.down
+        return (rows.shape[0] > GEMV_MAX_ROWS and context.shape == rows.shape
+                and context.dtype == rows.dtype
+                and rows.dtype in (torch.float16, torch.bfloat16)
+                and o.out_features == rows.shape[-1] == down.out_features
+                and o.smooth is None and o.static_scale is None
+                and type(o) is type(down) is W8A8Linear
+                and down.smooth is None and down.static_scale is None
+                and not any(m._forward_hooks or m._forward_pre_hooks for m in (o, down))
+                and not nn.modules.module._has_any_global_hook())
+
     @torch.no_grad()
     def forward(self, hidden_states: torch.Tensor, attention_state: Any = None) -> torch.Tensor:
         rows = _rows(hidden_states)
@@ -104,10 +125,15 @@ class W8A8LlamaLayer(nn.Module):
         # as one launch at decode shapes (w8a8_rmsnorm_linear).
         q, k, v = self.qkv.project_rmsnorm(rows, self.input_layernorm)
         context = self.attention_core(q, k, v, self.layer_index, attention_state)
-        attn_out = self.o_proj(context)
-        residual, mlp_out = self.mlp.forward_residual_rmsnorm(attn_out, rows,
-                                                              self.post_attention_layernorm)
-        out = residual + mlp_out
+        if self._adds_in_epilogues(context, rows):
+            summed = self.o_proj.forward_residual(context, rows, ss_parts=False).y
+            out = self.mlp.forward_rmsnorm_ss_residual(summed, None,
+                                                       self.post_attention_layernorm).y
+        else:
+            attn_out = self.o_proj(context)
+            residual, mlp_out = self.mlp.forward_residual_rmsnorm(attn_out, rows,
+                                                                  self.post_attention_layernorm)
+            out = residual + mlp_out
         return out.unsqueeze(0) if hidden_states.dim() == 3 else out
 
     @torch.no_grad()
