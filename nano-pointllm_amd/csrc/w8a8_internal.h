@@ -150,7 +150,7 @@ enum GemmTile : int {
 };
 int gemm_tile_choice(int64_t MB, int64_t NB, int64_t cus);
 
-// Pipelined GEMM tiles (gemm_pipe_kernel, 8 wavefronts, one workgroup per CU),
+// Pipelined GEMM tiles (gemm_pipe_kernel, 8 wavefronts unless said, one workgroup per CU),
 // taken before the ring tiles above: gemm_pipe_choice's answer for MB x NB
 // blocks over KB k-blocks (64 K), or kPipeNone.
 enum GemmPipe : int {
@@ -162,6 +162,10 @@ enum GemmPipe : int {
   kPipe192x288 = 4,
   kPipe256x256 = 5,
   kPipe256x352 = 6,
+  kPipe128x96 = 7,
+  kPipe128x64 = 8,
+  kPipe64x64 = 9,  // 4 wavefronts
+  kPipe192x352 = 10,
 };
 int gemm_pipe_choice(int64_t MB, int64_t NB, int64_t KB, int64_t cus);
 
@@ -174,6 +178,8 @@ hipError_t launch_gemv(const LinearOperands& op, hipStream_t st);
 bool gemv_tiles_supported(int64_t M, int64_t N, int64_t K, int epi, int y_dtype);
 // Any M; activations packed.
 hipError_t launch_gemm(const LinearOperands& op, hipStream_t st);
+// The same on pipelined tile `tile` (gemm_pipe_choice's answer for it).
+hipError_t launch_gemm_pipe(const LinearOperands& op, int tile, hipStream_t st);
 
 constexpr int64_t kGemvMaxRows = 64;
 

@@ -30,7 +30,8 @@ NOALLOC_SCRATCH_BYTES = 16 << 20
 GEMM_TILE_NAMES = ("tiny-deep", "small-deep", "big-deep", "big", "w192", "w224", "w256",
                    "w256sq", "mid", "wd7x2", "t112x96", "t128x96")
 # Names of the pipelined GEMM tiles w8a8_gemm_pipe_config returns, by code.
-GEMM_PIPE_NAMES = ("128x128", "192x160", "256x128", "256x192", "192x288", "256x256", "256x352")
+GEMM_PIPE_NAMES = ("128x128", "192x160", "256x128", "256x192", "192x288", "256x256", "256x352",
+                   "128x96", "128x64", "64x64", "192x352")
 
 _TORCH_TO_CODE = {
     torch.float32: F32,

@@ -12,12 +12,18 @@ import numpy as np
 import pytest
 import torch
 
+from gemm_tiles import gemm_config
 from oracle import w8a8_oracle as O
 
-SHAPES = [(130, 9870, 1030, "128x128"), (257, 12390, 1100, "192x160"),
+SHAPES = [(66, 4886, 1030, "64x64"), (65, 9858, 1100, "128x64"), (129, 8230, 1160, "128x96"),
+          (130, 12400, 1250, "128x128"), (257, 12390, 1100, "192x160"),
           (195, 20588, 1160, "256x128"), (260, 21950, 1250, "256x192"),
-          (513, 16350, 1030, "192x288"), (580, 18466, 1100, "256x256"),
-          (580, 21762, 1160, "256x352"), (600, 21770, 1250, "256x352")]
+          (515, 16350, 1030, "192x288"), (580, 18510, 1100, "256x256"),
+          (577, 21800, 1160, "192x352"), (580, 22570, 1250, "256x352")]
+# One shape per tile of the ring kernels, at a K that leaves it to them.
+RING = [(100, 1000, 900, "tiny-deep"), (300, 6000, 900, "small-deep"), (760, 4096, 900, "big-deep"),
+        (567, 12288, 300, "big"), (128, 4096, 900, "mid"), (560, 12288, 300, "wd7x2"),
+        (560, 4096, 900, "t112x96"), (640, 4096, 900, "t128x96")]
 
 
 def note(msg: str) -> None:
@@ -33,9 +39,10 @@ def pipe_config(m, n, k, cus=256):
 
 
 @pytest.mark.parametrize("m,n,k,tile", [(m, n, k, t) for m, n, k, t in SHAPES] + [
-    (560, 12288, 4096, "192x160"), (560, 22016, 4096, "192x288"), (560, 4096, 11008, "128x128"),
+    (560, 12288, 4096, "192x160"), (560, 22016, 4096, "192x288"), (560, 4096, 11008, "128x96"), (1024, 4096, 11008, "128x128"),
     (1024, 22016, 4096, "256x352"), (2048, 4096, 4096, "256x128"), (2048, 12288, 4096, "256x192"),
-    (448, 4096, 4096, None), (64, 22016, 8192, None), (2048, 12288, 960, None),
+    (201, 12288, 4096, "128x96"), (201, 4096, 4096, "64x64"), (448, 4096, 4096, "128x64"),
+    (768, 22016, 4096, "192x352"), (100, 4096, 11008, None), (64, 22016, 8192, None), (2048, 12288, 960, None),
     (0, 4096, 4096, None), (560, 4096, 0, None)])
 def test_rule(m, n, k, tile):
     assert pipe_config(m, n, k) == tile
@@ -54,12 +61,15 @@ def _case(m, n, k, dev):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("m,n,k,tile", SHAPES)
-def test_pipe_tile_int32_and_dequant(cuda, m, n, k, tile):
+@pytest.mark.parametrize("m,n,k,tile", SHAPES + RING)
+def test_tile_int32_and_dequant(cuda, m, n, k, tile):
     from nanopointllm_amd import w8a8
 
-    assert pipe_config(m, n, k) == tile
-    note(f"gemm pipe {tile} m={m} n={n} k={k}")
+    if k < 1024:
+        assert pipe_config(m, n, k) is None and gemm_config(m, n) == tile
+    else:
+        assert pipe_config(m, n, k) == tile
+    note(f"gemm {tile} m={m} n={n} k={k}")
     xq, wq, eacc, sx, sw, bias = _case(m, n, k, cuda)
     wp = w8a8.pack_rows(wq)
     np.testing.assert_array_equal(w8a8.gemm_i32(xq, wp, n).cpu().numpy(), eacc)

@@ -20,11 +20,10 @@ def note(msg: str) -> None:
     sys.__stderr__.flush()
 
 
-# ring mid / small / t112x96 / w256sq (K < 1024), pipelined 128x128, 192x160,
-# 256x128, 256x192 and 256x352
+# ring mid / small / t112x96 / w256sq (K < 1024), then pipelined tiles
 @pytest.mark.parametrize("m,n,k", [
     (65, 1000, 520), (300, 3001, 520), (560, 4096, 520), (2040, 16380, 136), (200, 12288, 1040),
-    (300, 12295, 1040), (2048, 4096, 1100), (520, 12000, 1040), (1024, 22016, 1024)])
+    (300, 12295, 1040), (2048, 4096, 1100), (520, 12000, 1040), (1024, 22016, 1024), (201, 4100, 1040), (350, 4096, 1100)])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_residual_in_gemm_epilogue(cuda, m, n, k, dtype):
     from nanopointllm_amd import w8a8
