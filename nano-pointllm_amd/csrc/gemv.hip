@@ -676,14 +676,16 @@ hipError_t launch_rows(const GemvParams& p, hipStream_t st) {
 
 // Ring shape by row tiles: two (M <= 32) stream steps of four k-blocks, three
 // in flight, or of two when a CU has a single block (O at M = 32: 7.4
-// against 8.1 us); four (M <= 64) one k-block per step, four in flight, to
-// keep the registers of the 16 x fragments.
+// against 8.1 us); three and four (M <= 48, 64) one k-block per step, four in
+// flight, to keep the registers of the 12 or 16 x fragments (a 4096 x 11008 MLP
+// call at 48 rows 46.7 us with three tiles, 47.2 with four).
 template <int EPI, typename TY, typename TH>
 hipError_t launch_rows_m(const GemvParams& p, hipStream_t st) {
   if (p.M <= 32)
     return p.NB > p.G ? launch_rows<2, 4, 3, EPI, TY, TH>(p, st)
                       : launch_rows<2, 2, 4, EPI, TY, TH>(p, st);
-  return launch_rows<4, 1, 4, EPI, TY, TH>(p, st);
+  return p.M <= 48 ? launch_rows<3, 1, 4, EPI, TY, TH>(p, st)
+                   : launch_rows<4, 1, 4, EPI, TY, TH>(p, st);
 }
 
 template <int NBW, int EPI, typename TY, typename TH>
