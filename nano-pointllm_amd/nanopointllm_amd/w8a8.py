@@ -167,6 +167,24 @@ def _workspace(m: int, k: int, device: torch.device) -> torch.Tensor:
     return torch.empty((max(workspace_bytes(m, k), 16),), dtype=torch.uint8, device=device)
 
 
+#: Most rows that any kernel quantizes inside its product (gemv_fused.hip).
+_FUSED_MAX_ROWS = 16
+
+
+def _call_with_workspace(fn, args: list, m: int, k: int, device: torch.device) -> int:
+    """``fn(*args, workspace, bytes, stream)``.  Decode shapes run fused and
+    need no workspace; the others report ERR_WORKSPACE (before any launch) and
+    are called again with one.  Past the fused kernels' rows every call needs
+    it, and the first call (2 to 3 us of a call of 25 at 201 rows) is left out."""
+    stream = _lib.stream_handle(device)
+    if m <= _FUSED_MAX_ROWS:
+        rc = fn(*args, None, 0, stream)
+        if rc != _lib.ERR_WORKSPACE:
+            return rc
+    ws = _workspace(m, k, device)
+    return fn(*args, ws.data_ptr(), ws.numel(), stream)
+
+
 def _check_operands(k: int, w_packed: torch.Tensor, w_scale: torch.Tensor | None,
                     bias: torch.Tensor | None, n: int, in_features: int | None) -> None:
     """Host checks before any launch: the C ABI only sees pointers, so an
@@ -248,14 +266,7 @@ def linear_dynamic(x: torch.Tensor, w_packed: torch.Tensor, w_scale: torch.Tenso
                 w_scale.data_ptr(), _lib.ptr(bias), epilogue, y.data_ptr(),
                 _lib.dtype_code(out_dtype), cols, float(y_scale), _lib.dtype_code(inter_dtype),
                 m, n, k, _lib.ptr(x_scale_out)]
-        stream = _lib.stream_handle(device)
-        # Decode shapes run fused and need no workspace; others report
-        # ERR_WORKSPACE (before any launch) and are retried with one.
-        rc = lib.w8a8_linear(*args, None, 0, stream)
-        if rc == _lib.ERR_WORKSPACE:
-            ws = _workspace(m, k, device)
-            rc = lib.w8a8_linear(*args, ws.data_ptr(), ws.numel(), stream)
-        _lib.check(rc, "w8a8_linear")
+        _lib.check(_call_with_workspace(lib.w8a8_linear, args, m, k, device), "w8a8_linear")
     return y.reshape(*x.shape[:-1], cols)
 
 
@@ -272,17 +283,12 @@ def _residual_rows(residual: torch.Tensor, m: int, n: int,
 
 
 def _residual_call(name: str, args: list, m: int, k: int, device, *, retry: bool) -> None:
-    lib = _lib.load()
-    stream = _lib.stream_handle(device)
-    fn = getattr(lib, name)
+    fn = getattr(_lib.load(), name)
     if retry:
-        rc = fn(*args, None, 0, stream)
-        if rc == _lib.ERR_WORKSPACE:
-            ws = _workspace(m, k, device)
-            rc = fn(*args, ws.data_ptr(), ws.numel(), stream)
+        rc = _call_with_workspace(fn, args, m, k, device)
     else:
         ws = _workspace(m, k, device)
-        rc = fn(*args, ws.data_ptr(), ws.numel(), stream)
+        rc = fn(*args, ws.data_ptr(), ws.numel(), _lib.stream_handle(device))
     _lib.check(rc, name)
 
 
@@ -591,7 +597,6 @@ def rmsnorm_linear(x: torch.Tensor, norm_weight: torch.Tensor, eps: float,
             raise ValueError("ss_parts must be float32 [rows, >= ceil(K/8)] RMSNorm chunk sums")
     if m and n:
         lib = _lib.load()
-        stream = _lib.stream_handle(device)
         if use_ss:
             name = "w8a8_rmsnorm_linear_ss"
             args = [x2.data_ptr(), _lib.dtype_code(x.dtype), ldx, ss_parts.data_ptr(),
@@ -606,12 +611,7 @@ def rmsnorm_linear(x: torch.Tensor, norm_weight: torch.Tensor, eps: float,
                     w_scale.data_ptr(), _lib.ptr(bias), epilogue, y.data_ptr(),
                     _lib.dtype_code(out_dtype), cols, float(y_scale), _lib.dtype_code(x.dtype),
                     m, n, k, None, _lib.ptr(rows), k]
-        fn = getattr(lib, name)
-        rc = fn(*args, None, 0, stream)
-        if rc == _lib.ERR_WORKSPACE:
-            ws = _workspace(m, k, device)
-            rc = fn(*args, ws.data_ptr(), ws.numel(), stream)
-        _lib.check(rc, name)
+        _lib.check(_call_with_workspace(getattr(lib, name), args, m, k, device), name)
     lead = x.shape[:-1]
     return NormLinearOutput(y.reshape(*lead, cols),
                             None if res_out is None else res_out.reshape(x.shape),
