@@ -153,6 +153,10 @@ __global__ __launch_bounds__(WM * WN * 64, OCC * WM * WN / 4) void gemm_kernel(G
     }
   }
 
+  if (NS == 0) {  // K = 0: no stage's barrier has stood behind the scales' copies
+    wait_vmcnt<0>();
+    ring_barrier();
+  }
   store_tile<WM, WN, BR, BC, kRing, EPI, TY, TH>(p, acc, wm, wn, mb0, nb0, lane, smem, scales);
 }
 

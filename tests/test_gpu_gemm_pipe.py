@@ -111,3 +111,25 @@ def test_pipe_tile_silu_and_integer_epilogues(cuda, m, n, k, tile):
     y = E.linear_i8in_requant(xq, wp, mult, shift, bias, n)
     ref = E.requantize_int32(torch.from_numpy(eacc).to(cuda), bias, mult, shift)
     assert torch.equal(y, ref)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n", [(100, 1000), (300, 6000), (760, 4096), (560, 12288), (560, 4096)])
+def test_empty_reduction_gives_the_bias(cuda, m, n):
+    """K = 0 through the C ABI: no k-block's barrier stands between the copies
+    of the scales and bias to LDS and the epilogue that reads them."""
+    from nanopointllm_amd import _lib
+
+    note(f"gemm K = 0 m={m} n={n}")
+    lib = _lib.load()
+    xq = torch.zeros(m, 16, dtype=torch.int8, device=cuda)
+    sx, sw = torch.full((m,), 0.5, device=cuda), torch.full((n,), 0.25, device=cuda)
+    bias = torch.randn(n, generator=torch.Generator().manual_seed(n)).to(cuda)
+    y = torch.full((m, n), 7.0, dtype=torch.float16, device=cuda)
+    ws = torch.empty(max(256, lib.w8a8_workspace_bytes(m, 0)), dtype=torch.uint8, device=cuda)
+    rc = lib.w8a8_linear_i8in(xq.data_ptr(), 16, sx.data_ptr(), None, sw.data_ptr(),
+                              bias.data_ptr(), _lib.EPI_DEQUANT, y.data_ptr(), _lib.F16, n, 0.0,
+                              _lib.F16, m, n, 0, ws.data_ptr(), ws.numel(),
+                              _lib.stream_handle(cuda))
+    _lib.check(rc, "w8a8_linear_i8in")
+    assert torch.equal(y, bias.half().expand(m, n))
