@@ -62,7 +62,10 @@ __device__ inline i32x4 mfma_16x16x64(i32x4 a, i32x4 b, i32x4 c) {
 // requested before the weights so that the epilogue does not wait a memory
 // round trip for them.  Clamped addresses: the outputs they stand for past M
 // or N are not written.
-template <typename TY>
+// SCALES: the row and column scales too (gemv_tiles_kernel; in gemv_kernel at
+// 3 rows they delayed the weights by more than the epilogue gained, 0.6 of 48 us
+// of an MLP).
+template <typename TY, bool SCALES>
 struct FirstOutput {
   TY res{};
   float sx = 0.0f, sw = 0.0f;
@@ -73,8 +76,10 @@ struct FirstOutput {
       const int m = min(((e % (MT * 256)) >> 8) * 16 + ((e & 255) >> 4), p.M - 1);
       const int64_t nc = (nb0 + e / (MT * 256)) * 16 + (e & 15);
       const int64_t n = nc < p.N ? nc : p.N - 1;
-      sx = p.sx[m];
-      sw = p.sw[n];
+      if constexpr (SCALES) {
+        sx = p.sx[m];
+        sw = p.sw[n];
+      }
       if (p.res != nullptr) res = static_cast<const TY*>(p.res)[m * p.ld_res + n];
     }
   }
@@ -83,13 +88,13 @@ struct FirstOutput {
 // Sums the wavefronts' int32 partials red[w][j * 256 MT + 256 mt + 16 row +
 // column] (complete: the caller has passed a barrier) and writes the NBW
 // blocks' outputs through the epilogue EPI.
-template <int WAVES, int MT, int NBW, int EPI, typename TY, typename TH>
+template <int WAVES, int MT, int NBW, int EPI, typename TY, typename TH, bool SCALES>
 __device__ inline void gemv_store(const GemvParams& p, const int32_t (*red)[NBW * MT * 256],
-                                  int64_t nb0, int tid, const FirstOutput<TY>& first) {
+                                  int64_t nb0, int tid, const FirstOutput<TY, SCALES>& first) {
   constexpr int NT = WAVES * 64;
   constexpr int TB = MT * 256;  // int32 partials of one block per wave
   [[maybe_unused]] auto dequant = [&](int32_t s, int e, int m, int64_t n) {
-    const bool f = e == tid;
+    const bool f = SCALES && e == tid;
     return dequant1(s, f ? first.sx : p.sx[m], f ? first.sw : p.sw[n], p.bias, n);
   };
   if constexpr (EPI == kEpiI32 || EPI == kEpiDequant || EPI == kEpiRequant ||
@@ -223,7 +228,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_kernel(GemvParams p) {
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) acc[j][mt] = i32x4{0, 0, 0, 0};
 
-  FirstOutput<TY> first;
+  FirstOutput<TY, false> first;
   first.template load<MT, NBW, EPI>(p, nb0, tid);
 
   i32x4 wb0[NBW][CH], wb1[NBW][CH];
@@ -573,7 +578,7 @@ __global__ __launch_bounds__(kRowsThreads) void gemv_rows_kernel(GemvParams p) {
 }
 
 // Activations already in the packed 16x64 tiles (gemv_tiles_kernel): K > 4096
-// with few output blocks (down at 17..64 rows, and at 9..16 where the fused
+// with few output blocks (down at 17..64 rows, and wide ones at 9..16 where the fused
 // kernels do not reach).  One workgroup of 16 wavefronts per NBW blocks, one
 // workgroup per CU; the wavefronts split K, and each streams its k-blocks of
 // the NBW weight blocks and MT activation tiles through a ring of D register
@@ -610,7 +615,7 @@ __global__ __launch_bounds__(1024) void gemv_tiles_kernel(GemvParams p) {
   const int nk = KB * (wave + 1) / WAVES - kb0;
   const int MB = (p.M + 15) / 16;
 
-  FirstOutput<TY> first;
+  FirstOutput<TY, true> first;
   first.template load<MT, NBW, EPI>(p, nb0, tid);
 
   // Blocks past the last one re-read it (their products are not stored).
@@ -759,8 +764,11 @@ bool gemv_rows_supported(int64_t M, int64_t N, int64_t K, int64_t lda, int epi) 
 
 bool gemv_tiles_supported(int64_t M, int64_t N, int64_t K, int epi, int y_dtype) {
   const bool typed = epi == kEpiI32 || (epi == kEpiDequant && (y_dtype == kF16 || y_dtype == kBF16));
-  return typed && M > 8 && M <= kGemvMaxRows && K > 4096 &&
-         K < (int64_t{1} << 30) && ceil_div(N, kTileRows) <= 2 * cu_count();
+  const int64_t nb = ceil_div(N, kTileRows);
+  // Up to 16 rows with one block per CU gemv_kernel is level (13 rows, 4096 x
+  // 10464 MLP: 33.4 against 33.7 us): its rows are few and its grid is even.
+  return typed && M > 8 && M <= kGemvMaxRows && (M > 16 || nb > cu_count()) && K > 4096 &&
+         K < (int64_t{1} << 30) && nb <= 2 * cu_count();
 }
 
 hipError_t launch_gemv(const LinearOperands& op, hipStream_t st) {

@@ -172,7 +172,8 @@ int gemm_pipe_choice(int64_t MB, int64_t NB, int64_t KB, int64_t cus);
 // M <= 64 (the GEMV regime).
 hipError_t launch_gemv(const LinearOperands& op, hipStream_t st);
 // Whether the GEMV takes this product's activations in the packed tiles
-// (op.a_tiles): int32 or 16-bit dequant outputs, 9..64 rows, K > 4096 and at
+// (op.a_tiles): int32 or 16-bit dequant outputs, K > 4096, 17..64 rows (9..16
+// where there are more output blocks than CUs) and at
 // most two output blocks per CU.  Callers that write the activations
 // themselves then write tiles.
 bool gemv_tiles_supported(int64_t M, int64_t N, int64_t K, int epi, int y_dtype);

@@ -1,6 +1,6 @@
 """The GEMV on activations in the packed tiles (csrc/gemv.hip
-``gemv_tiles_kernel``): 9..64 rows, K > 4096, at most two output blocks per CU,
-where the library quantizes the rows itself.  Bit-equal to the general route,
+``gemv_tiles_kernel``): 17..64 rows (9..16 with more output blocks than CUs),
+K > 4096, at most two output blocks per CU, where the library quantizes the rows itself.  Bit-equal to the general route,
 the same int8 rows handed over row-major (``gemv_kernel``), at every count of
 row tiles, one and two blocks per workgroup, ragged N, K of uneven wavefront
 shares and off the 64-column grid, strided x, bias, int32 and both 16-bit
@@ -35,10 +35,10 @@ def _case(m, n, k, dtype, dev, pad=0):
     return x, wq, w8a8.pack_rows(wq.to(dev)), sw, bias
 
 
-# (m, n, k): 9 and 64 are the rule's ends, 16/17, 32/33 and 48/49 those of the
+# (m, n, k): 9 (at 5120 outputs) and 64 are the rule's ends, 16/17, 32/33 and 48/49 those of the
 # row tiles; 4096 outputs give one block per CU, 4100 and 5120 two, 8192 the most.
 @pytest.mark.parametrize("m,n,k", [
-    (9, 4096, 11008), (16, 5120, 13824), (17, 4096, 4104), (32, 4100, 4160), (33, 8192, 4168),
+    (9, 5120, 11008), (16, 4096, 11008), (16, 5120, 13824), (17, 4096, 4104), (32, 4100, 4160), (33, 8192, 4168),
     (48, 4096, 11008), (49, 5120, 6400), (64, 4096, 11008), (64, 40, 8200), (12, 8, 16384)])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_tiles_match_row_major_route(cuda, m, n, k, dtype):
