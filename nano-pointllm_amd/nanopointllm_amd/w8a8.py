@@ -168,21 +168,13 @@ def _workspace(m: int, k: int, device: torch.device) -> torch.Tensor:
 
 
 #: Most rows that any kernel quantizes inside its product (gemv_fused.hip).
+#: Up to here an entry point is first called without a workspace: fused shapes
+#: need none, the others report ERR_WORKSPACE before any launch and are called
+#: again with one.  Past them every call needs it and makes one call (2 to 3 us
+#: of a call of 25 at 201 rows).  Each wrapper spells the two calls out: a
+#: helper's frame between it and the library is 0.1 us of a decode call of 12
+#: that the host bounds.
 _FUSED_MAX_ROWS = 16
-
-
-def _call_with_workspace(fn, args: list, m: int, k: int, device: torch.device) -> int:
-    """``fn(*args, workspace, bytes, stream)``.  Decode shapes run fused and
-    need no workspace; the others report ERR_WORKSPACE (before any launch) and
-    are called again with one.  Past the fused kernels' rows every call needs
-    it, and the first call (2 to 3 us of a call of 25 at 201 rows) is left out."""
-    stream = _lib.stream_handle(device)
-    if m <= _FUSED_MAX_ROWS:
-        rc = fn(*args, None, 0, stream)
-        if rc != _lib.ERR_WORKSPACE:
-            return rc
-    ws = _workspace(m, k, device)
-    return fn(*args, ws.data_ptr(), ws.numel(), stream)
 
 
 def _check_operands(k: int, w_packed: torch.Tensor, w_scale: torch.Tensor | None,
@@ -266,7 +258,12 @@ def linear_dynamic(x: torch.Tensor, w_packed: torch.Tensor, w_scale: torch.Tenso
                 w_scale.data_ptr(), _lib.ptr(bias), epilogue, y.data_ptr(),
                 _lib.dtype_code(out_dtype), cols, float(y_scale), _lib.dtype_code(inter_dtype),
                 m, n, k, _lib.ptr(x_scale_out)]
-        _lib.check(_call_with_workspace(lib.w8a8_linear, args, m, k, device), "w8a8_linear")
+        stream = _lib.stream_handle(device)
+        rc = lib.w8a8_linear(*args, None, 0, stream) if m <= _FUSED_MAX_ROWS else _lib.ERR_WORKSPACE
+        if rc == _lib.ERR_WORKSPACE:
+            ws = _workspace(m, k, device)
+            rc = lib.w8a8_linear(*args, ws.data_ptr(), ws.numel(), stream)
+        _lib.check(rc, "w8a8_linear")
     return y.reshape(*x.shape[:-1], cols)
 
 
@@ -284,11 +281,11 @@ def _residual_rows(residual: torch.Tensor, m: int, n: int,
 
 def _residual_call(name: str, args: list, m: int, k: int, device, *, retry: bool) -> None:
     fn = getattr(_lib.load(), name)
-    if retry:
-        rc = _call_with_workspace(fn, args, m, k, device)
-    else:
+    stream = _lib.stream_handle(device)
+    rc = fn(*args, None, 0, stream) if retry and m <= _FUSED_MAX_ROWS else _lib.ERR_WORKSPACE
+    if rc == _lib.ERR_WORKSPACE:
         ws = _workspace(m, k, device)
-        rc = fn(*args, ws.data_ptr(), ws.numel(), _lib.stream_handle(device))
+        rc = fn(*args, ws.data_ptr(), ws.numel(), stream)
     _lib.check(rc, name)
 
 
@@ -611,7 +608,13 @@ def rmsnorm_linear(x: torch.Tensor, norm_weight: torch.Tensor, eps: float,
                     w_scale.data_ptr(), _lib.ptr(bias), epilogue, y.data_ptr(),
                     _lib.dtype_code(out_dtype), cols, float(y_scale), _lib.dtype_code(x.dtype),
                     m, n, k, None, _lib.ptr(rows), k]
-        _lib.check(_call_with_workspace(getattr(lib, name), args, m, k, device), name)
+        fn = getattr(lib, name)
+        stream = _lib.stream_handle(device)
+        rc = fn(*args, None, 0, stream) if m <= _FUSED_MAX_ROWS else _lib.ERR_WORKSPACE
+        if rc == _lib.ERR_WORKSPACE:
+            ws = _workspace(m, k, device)
+            rc = fn(*args, ws.data_ptr(), ws.numel(), stream)
+        _lib.check(rc, name)
     lead = x.shape[:-1]
     return NormLinearOutput(y.reshape(*lead, cols),
                             None if res_out is None else res_out.reshape(x.shape),
