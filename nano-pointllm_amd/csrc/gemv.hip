@@ -60,36 +60,45 @@ __device__ inline i32x4 mfma_16x16x64(i32x4 a, i32x4 b, i32x4 c) {
 // The operands of the output a thread of gemv_kernel or gemv_tiles_kernel
 // writes first (element e == tid of the workgroup's NBW blocks x MT row tiles),
 // requested before the weights so that the epilogue does not wait a memory
-// round trip for them.  Clamped addresses: the outputs they stand for past M
-// or N are not written.
-// SCALES: the row and column scales too (gemv_tiles_kernel; in gemv_kernel at
-// 3 rows they delayed the weights by more than the epilogue gained, 0.6 of 48 us
-// of an MLP).
+// round trip for them (later outputs, when a thread has several, load then).
+// SCALES (gemv_tiles_kernel): the row and column scales too, from clamped
+// addresses, the outputs they stand for past M or N being unwritten.  In
+// gemv_kernel, whose wavefronts have less to do before their first weights,
+// the scales cost more there than the epilogue gains (0.6 of 48 us of an MLP
+// at 3 rows), so it takes only the residual, behind its bounds check.
 template <typename TY, bool SCALES>
 struct FirstOutput {
   TY res{};
   float sx = 0.0f, sw = 0.0f;
   template <int MT, int NBW, int EPI>
   __device__ inline void load(const GemvParams& p, int64_t nb0, int tid) {
-    if constexpr (EPI == kEpiDequant) {
-      const int e = tid < NBW * MT * 256 ? tid : 0;
-      const int m = min(((e % (MT * 256)) >> 8) * 16 + ((e & 255) >> 4), p.M - 1);
-      const int64_t nc = (nb0 + e / (MT * 256)) * 16 + (e & 15);
+    constexpr int TB = MT * 256;
+    if constexpr (EPI == kEpiDequant && SCALES) {
+      const int e = tid < NBW * TB ? tid : 0;
+      const int m = min(((e % TB) >> 8) * 16 + ((e & 255) >> 4), p.M - 1);
+      const int64_t nc = (nb0 + e / TB) * 16 + (e & 15);
       const int64_t n = nc < p.N ? nc : p.N - 1;
-      if constexpr (SCALES) {
-        sx = p.sx[m];
-        sw = p.sw[n];
-      }
+      sx = p.sx[m];
+      sw = p.sw[n];
       if (p.res != nullptr) res = static_cast<const TY*>(p.res)[m * p.ld_res + n];
+    } else if constexpr (EPI == kEpiDequant) {
+      if (p.res != nullptr && tid < NBW * TB) {
+        const int m = ((tid % TB) >> 8) * 16 + ((tid & 255) >> 4);
+        const int64_t nb = nb0 + tid / TB;
+        const int64_t n = nb * 16 + (tid & 15);
+        if (m < p.M && nb < p.NB && n < p.N) res = static_cast<const TY*>(p.res)[m * p.ld_res + n];
+      }
     }
   }
 };
 
 // Sums the wavefronts' int32 partials red[w][j * 256 MT + 256 mt + 16 row +
 // column] (complete: the caller has passed a barrier) and writes the NBW
-// blocks' outputs through the epilogue EPI.
+// blocks' outputs through the epilogue EPI.  p is a copy: by reference (and with
+// clamped residual addresses) gemv_kernel's dequant form took 4 registers more
+// and reached its first weights later, 3 x 5120 x 13824 21.1 us a call, not 20.8.
 template <int WAVES, int MT, int NBW, int EPI, typename TY, typename TH, bool SCALES>
-__device__ inline void gemv_store(const GemvParams& p, const int32_t (*red)[NBW * MT * 256],
+__device__ inline void gemv_store(const GemvParams p, const int32_t (*red)[NBW * MT * 256],
                                   int64_t nb0, int tid, const FirstOutput<TY, SCALES>& first) {
   constexpr int NT = WAVES * 64;
   constexpr int TB = MT * 256;  // int32 partials of one block per wave
@@ -103,11 +112,11 @@ __device__ inline void gemv_store(const GemvParams& p, const int32_t (*red)[NBW 
       const int m = ((e % TB) >> 8) * 16 + ((e & 255) >> 4);
       const int64_t nb = nb0 + e / TB;
       const int64_t n = nb * 16 + (e & 15);
+      const bool ok = m < p.M && nb < p.NB && n < p.N;
       if constexpr (EPI == kEpiDequant) {
         if (p.res != nullptr) {
           // Residual-add epilogue: the chunk sums need every lane, so no lane
           // leaves before them (NBW * TB and NT are multiples of 64).
-          const bool ok = m < p.M && nb < p.NB && n < p.N;
           float v = 0.0f;
           if (ok) {
             int32_t s = 0;
@@ -125,7 +134,7 @@ __device__ inline void gemv_store(const GemvParams& p, const int32_t (*red)[NBW 
           continue;
         }
       }
-      if (m >= p.M || nb >= p.NB || n >= p.N) continue;
+      if (!ok) continue;
       int32_t s = 0;
 #pragma unroll
       for (int w = 0; w < WAVES; ++w) s += red[w][e];
