@@ -61,6 +61,9 @@ from .linear import W8A8Linear, W8A8MLP, W8A8PackedQKV, _norm_eps
 #: Most rows the GEMV kernels take (kGemvMaxRows).
 GEMV_MAX_ROWS = 64
 
+#: Calls of o_proj, the MLP and its down that the layer's epilogue route replaces.
+_REPLACED_CALLS = frozenset(("forward", "forward_i8", "forward_residual_rmsnorm"))
+
 AttentionCore = Callable[[torch.Tensor, torch.Tensor, torch.Tensor, int, Any], torch.Tensor]
 
 
@@ -105,16 +108,20 @@ class W8A8LlamaLayer(nn.Module):
         past the GEMV's rows, where the GEMM adds them as it writes (at fewer
         rows the plain kernels are the faster ones), for 16-bit rows of one
         dtype, per-token o_proj activations, and modules whose calls nothing
-        observes (the epilogue route goes past ``__call__`` and its hooks).
+        observes or replaces (the epilogue route goes past ``__call__`` and its
+        hooks, past a subclass's methods and past an instance's own ones).
         The bits are the same: one rounding of the sum either way."""
-        o, down = self.o_proj, self.mlp.down
-        return (rows.shape[0] > GEMV_MAX_ROWS and context.shape == rows.shape
+        o, mlp = self.o_proj, self.mlp
+        if rows.shape[0] <= GEMV_MAX_ROWS or type(o) is not W8A8Linear or type(mlp) is not W8A8MLP:
+            return False
+        down = mlp.down
+        return (type(down) is W8A8Linear and context.shape == rows.shape
                 and context.dtype == rows.dtype
                 and rows.dtype in (torch.float16, torch.bfloat16)
                 and o.out_features == rows.shape[-1] == down.out_features
                 and o.smooth is None and o.static_scale is None
-                and type(o) is type(down) is W8A8Linear
                 and down.smooth is None and down.static_scale is None
+                and all(_REPLACED_CALLS.isdisjoint(vars(m)) for m in (o, mlp, down))
                 and not any(m._forward_hooks or m._forward_pre_hooks for m in (o, down))
                 and not nn.modules.module._has_any_global_hook())
 
