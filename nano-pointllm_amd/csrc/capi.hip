@@ -508,7 +508,7 @@ int w8a8_quant_rows(const void* x, int x_dtype, int64_t rows, int64_t k, int64_t
 int w8a8_qdq_rows(const void* x, int x_dtype, int64_t rows, int64_t k, int64_t ldx, int64_t group,
                   int8_t* q, int64_t ldq, void* deq, int64_t ld_deq, float* scales,
                   hipStream_t stream) {
-  if (rows < 0 || k < 0 || rows > kMaxRows || k > kMaxRows || group < 0) return W8A8_ERR_SHAPE;
+  if (rows < 0 || k < 0 || rows > kMaxRows || group < 0) return W8A8_ERR_SHAPE;
   if (!float_dtype(x_dtype)) return W8A8_ERR_DTYPE;
   if (rows == 0 || k == 0) return W8A8_OK;
   if (x == nullptr || deq == nullptr || scales == nullptr) return W8A8_ERR_NULL;

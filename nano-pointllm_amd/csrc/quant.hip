@@ -809,6 +809,11 @@ void qdq_rows_launch(dim3 g, hipStream_t st, const TX* x, int64_t ldx, int64_t K
 #undef W8A8_QDQ_REG
 }
 
+// qdq_groups_kernel counts a row's chunks and groups in 32 bits (the 2^30 and
+// fewer of this K leave room for its last workgroup's idle lanes); the other
+// kernel's columns are 64-bit throughout.
+constexpr int64_t kQdqGroupsMaxK = int64_t{1} << 33;
+
 // Groups of 8, 16, .. 512 columns run on qdq_groups_kernel; other groups take
 // a workgroup each: one wavefront up to 512 columns, 256 threads past that.
 template <typename TX>
@@ -821,7 +826,8 @@ hipError_t qdq_dispatch(const TX* x, int64_t ldx, int64_t rows, int64_t K, int64
   out.vec_q = cols8 && aligned8(o.q) && o.ldq % 8 == 0;
   out.vec_d = cols8 && aligned16(o.deq) && o.ldd % 8 == 0;
   const int64_t lanes = group / 8;
-  if (group % 8 == 0 && lanes <= 64 && (lanes & (lanes - 1)) == 0 && groups > 1) {
+  if (group % 8 == 0 && lanes <= 64 && (lanes & (lanes - 1)) == 0 && groups > 1 &&
+      K <= kQdqGroupsMaxK) {
     const int64_t bpr = ceil_div(groups * lanes, kQuantThreads);
     if (rows * bpr > INT32_MAX) return hipErrorInvalidConfiguration;
 #define W8A8_QDQ_LPG(L)                                                                        \

@@ -112,3 +112,35 @@ def test_other_weight_types_go_through_binary32(cuda):
     want = w8a8.groupwise_weight_qdq(w.to(cuda), group_size=64)
     assert deq.dtype == torch.float64 and torch.equal(deq, want[0].double())
     assert torch.equal(q, want[1]) and torch.equal(s, want[2])
+
+
+def test_rows_past_32_bit_columns(cuda):
+    """One row of 2^31 + 8 columns: every index past 32 bits, against the same
+    columns of a short row with the same scale, at both ends and around the
+    signed and unsigned 32-bit boundaries of bytes and elements."""
+    from nanopointllm_amd import w8a8
+
+    k, n = (1 << 31) + 8, 4096
+    note(f"qdq one row of {k}")
+    x = torch.empty((1, k), dtype=torch.bfloat16, device=cuda)
+    x.copy_(torch.arange(8191, device=cuda).sub_(4095).to(torch.bfloat16)
+            .repeat(k // 8191 + 1)[None, :k])
+    x[0, 5] = 6000.0  # the row's largest, in the first slice
+    for group in (None, 128):
+        if group is None:
+            deq, s = w8a8.dynamic_per_token_activation_qdq(x)
+        else:
+            deq, q, s = w8a8.groupwise_weight_qdq(x, group_size=group)
+        for start in (0, (1 << 30) - n // 2, k - n - 8):
+            part = x[:, start:start + n].clone()
+            if group is None:
+                part = torch.cat([part, x[:, 5:6]], dim=1)
+                want, ws = w8a8.dynamic_per_token_activation_qdq(part)
+                assert torch.equal(s, ws)
+            else:
+                want, wq, ws = w8a8.groupwise_weight_qdq(part, group_size=group)
+                assert torch.equal(q[:, start:start + n], wq)
+                assert torch.equal(s[:, start // group:(start + n) // group], ws)
+            assert torch.equal(deq[:, start:start + n], want[:, :n])
+        del deq
+    assert s.shape == (1, k // 128 + 1)
