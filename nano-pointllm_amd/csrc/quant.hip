@@ -368,7 +368,9 @@ __global__ __launch_bounds__(kQuantThreads) void qdq_groups_kernel(
 // thread between the absmax and the outputs (REG 0: it is read twice).
 // Latency-bound at activation sizes: 560 x 4096 bfloat16 as a call takes 15.2
 // us, mostly the host's, against 31.2 for quant_rows_kernel (4.8 us) and three
-// elementwise passes (20 us).
+// elementwise passes (20 us).  Few long rows are bound by what one CU keeps in
+// flight, hence the four chunks at a time: one row of 2 million bfloat16 takes
+// 290 us (a chunk at a time on 512 threads 599, the separate kernels 366).
 template <typename TX, int REG, int NT>
 __global__ __launch_bounds__(NT) void qdq_rows_kernel(const TX* __restrict__ x, int64_t ldx,
                                                       int64_t K, int64_t group, int vec_in,
@@ -384,6 +386,27 @@ __global__ __launch_bounds__(NT) void qdq_rows_kernel(const TX* __restrict__ x, 
   out.deq = static_cast<TX*>(out.deq) + c0;
   const int64_t nchunk = (n + 7) / 8;
   auto valid_of = [&](int64_t k0) { return static_cast<int>(n - k0 <= 0 ? 0 : (n - k0 < 8 ? n - k0 : 8)); };
+  // REG 0: f(k0, valid columns, values) for each of the thread's chunks, four
+  // whole ones at a time so that their loads are in flight together.
+  [[maybe_unused]] auto each_chunk = [&](auto&& f) __attribute__((always_inline)) {
+    int64_t c = tid;
+    auto whole = [&](auto vec) __attribute__((always_inline)) {
+      for (; c + 3 * NT < n / 8; c += 4 * NT) {
+        float t[4][8];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) load8(xr + (c + u * NT) * 8, t[u], decltype(vec)::value, 8);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) f((c + u * NT) * 8, 8, t[u]);
+      }
+    };
+    if (vec_in) whole(std::true_type{}); else whole(std::false_type{});
+    for (; c < nchunk; c += NT) {
+      const int valid = valid_of(c * 8);
+      float t[8];
+      load8(xr + c * 8, t, vec_in != 0, valid);
+      f(c * 8, valid, t);
+    }
+  };
   float v[REG > 0 ? REG : 1][8];
   float amax = 0.0f;
   if constexpr (REG > 0) {
@@ -401,11 +424,10 @@ __global__ __launch_bounds__(NT) void qdq_rows_kernel(const TX* __restrict__ x, 
 #pragma unroll
       for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(v[c][j]));
   } else {
-    for (int64_t c = tid; c < nchunk; c += NT) {
-      load8(xr + c * 8, v[0], vec_in != 0, valid_of(c * 8));
+    each_chunk([&](int64_t, int, const float(&t)[8]) __attribute__((always_inline)) {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(v[0][j]));
-    }
+      for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(t[j]));
+    });
   }
   amax = wave_max_abs(amax);
   if constexpr (NT > 64) {
@@ -426,11 +448,9 @@ __global__ __launch_bounds__(NT) void qdq_rows_kernel(const TX* __restrict__ x, 
       if (valid > 0) qdq_store8<TX>(out, row, k0, valid, v[c], s, r);
     }
   } else {
-    for (int64_t c = tid; c < nchunk; c += NT) {
-      const int valid = valid_of(c * 8);
-      load8(xr + c * 8, v[0], vec_in != 0, valid);
-      qdq_store8<TX>(out, row, c * 8, valid, v[0], s, r);
-    }
+    each_chunk([&](int64_t k0, int valid, const float(&t)[8]) __attribute__((always_inline)) {
+      qdq_store8<TX>(out, row, k0, valid, t, s, r);
+    });
   }
 }
 
@@ -815,7 +835,11 @@ void qdq_rows_launch(dim3 g, hipStream_t st, const TX* x, int64_t ldx, int64_t K
 constexpr int64_t kQdqGroupsMaxK = int64_t{1} << 33;
 
 // Groups of 8, 16, .. 512 columns run on qdq_groups_kernel; other groups take
-// a workgroup each: one wavefront up to 512 columns, 256 threads past that.
+// a workgroup each: one wavefront up to 512 columns, 256 threads past that, 512
+// where up to 2048 workgroups leave the CUs room for them, and 1024 where there
+// are at most two workgroups per CU of more columns than 512 threads hold in
+// registers (one row of 70000 bfloat16 15.2 us a call, 18.2 on 512 threads;
+// 64 rows 15.1 against 21.7).
 template <typename TX>
 hipError_t qdq_dispatch(const TX* x, int64_t ldx, int64_t rows, int64_t K, int64_t group,
                         const QdqOut& o, float* scales, hipStream_t st) {
@@ -854,6 +878,8 @@ hipError_t qdq_dispatch(const TX* x, int64_t ldx, int64_t rows, int64_t K, int64
   const int ng = static_cast<int>(groups);
   if (n <= 512)
     qdq_rows_launch<TX, 64>(g, st, x, ldx, K, group, vec_in, ng, out, scales);
+  else if (rows * groups <= 2 * cu_count() && n > 8 * kRegChunksMax * 2 * kQuantThreads)
+    qdq_rows_launch<TX, 4 * kQuantThreads>(g, st, x, ldx, K, group, vec_in, ng, out, scales);
   else if (rows * groups <= 2048 && n > 8 * kQuantThreads)
     qdq_rows_launch<TX, 2 * kQuantThreads>(g, st, x, ldx, K, group, vec_in, ng, out, scales);
   else

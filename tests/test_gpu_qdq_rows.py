@@ -71,6 +71,26 @@ def test_rows_exact(cuda, m, k, dtype):
     assert torch.equal(deq.cpu(), rounded(edeq, dtype))
 
 
+# Per workgroup size (256, 512, 1024 threads): the last columns that stay in
+# registers, the first that are read twice, one whole round of four chunks a
+# thread and the columns behind it, aligned and not.
+@pytest.mark.parametrize("m,k", [(2049, 16384), (2049, 16392), (2049, 16391), (513, 32768),
+                                 (513, 32776), (515, 32769), (512, 32776), (1, 65536), (2, 65544),
+                                 (1, 65543), (2, 98304), (1, 98312), (1, 131071), (3, 300001)])
+@pytest.mark.parametrize("dtype", DTYPES, ids=str)
+def test_long_rows_equal_the_separate_kernels(cuda, m, k, dtype):
+    from nanopointllm_amd import w8a8
+
+    note(f"qdq long rows {m}x{k} {dtype}")
+    g = torch.Generator(device=cuda).manual_seed(m + k)
+    x = torch.empty((m, k), device=cuda, dtype=dtype).normal_(generator=g)
+    x[:, k - 1] = 9.0   # the last column holds the scale
+    q, s = w8a8.quant_rows(x)
+    deq, q2, s2 = w8a8.per_output_weight_qdq(x)
+    assert torch.equal(q2, q) and torch.equal(s2, s)
+    assert torch.equal(deq, (q.float() * s[:, None]).to(dtype))
+
+
 @pytest.mark.parametrize("group", [64, 96, 4096])
 def test_strided_and_unaligned_rows(cuda, group):
     from nanopointllm_amd import w8a8
