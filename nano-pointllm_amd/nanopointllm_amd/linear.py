@@ -38,6 +38,20 @@ from . import _lib
 from . import w8a8 as _w
 
 
+def _packs_in_one_kernel(weights: list[torch.Tensor], n: int) -> bool:
+    """Whether the kernel that quantizes straight into the packed tiles is the
+    faster one for these matrices of n rows in all.  It has a wavefront per row
+    and a workgroup per 16: a few rows past 32 KB keep too few CUs busy for too
+    long (48 x 65536 binary16 123 us, quantizing and packing apart 27), and a
+    single matrix whose rows it reads twice loses against them while they read
+    it once (up to 16384 columns; 5120 x 13824 binary16 68 us against 61, 4096 x
+    11008 binary32 61 against 54).  Several matrices would be concatenated first."""
+    k, es = weights[0].shape[1], weights[0].element_size()
+    if n <= 1024 and k * es > 32 << 10:
+        return False
+    return len(weights) > 1 or k <= (11264 if es == 2 else 4096) or (es == 2 and k > 16384)
+
+
 @dataclass
 class PackedW8A8Weight:
     """Per-output int8 weight in packed tiles, with f32 scales and bias."""
@@ -81,8 +95,9 @@ class PackedW8A8Weight:
                    layout: int = _lib.ROWS_AS_IS) -> "PackedW8A8Weight":
         """:meth:`from_float` of the matrices concatenated by rows, quantized
         straight into the packed tiles by one kernel.  Matrices that it does
-        not take (mixed types or devices, empty or unequal halves) are
-        concatenated and go through int8 rows."""
+        not take (mixed types or devices, empty or unequal halves) or is not
+        the faster one for (:func:`_packs_in_one_kernel`) are concatenated and
+        go through int8 rows."""
         weights = [w.detach() for w in weights]
         first = weights[0]
         n = sum(w.shape[0] for w in weights)
@@ -91,7 +106,8 @@ class PackedW8A8Weight:
         if not (0 < len(weights) <= 3 and first.dim() == 2 and first.numel()
                 and all(w.dim() == 2 and w.shape[1] == first.shape[1] and w.dtype == first.dtype
                         and w.device == first.device for w in weights)
-                and (layout == _lib.ROWS_AS_IS or (n % 2 == 0 and halves))):
+                and (layout == _lib.ROWS_AS_IS or (n % 2 == 0 and halves))
+                and _packs_in_one_kernel(weights, n)):
             q, s = _w.quant_rows(first if len(weights) == 1 else torch.cat(weights, dim=0))
             return cls.from_int8(q, s, bias, layout=layout)
         device = _lib.require_cuda(*weights, bias)

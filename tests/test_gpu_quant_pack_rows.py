@@ -65,6 +65,50 @@ def test_equals_quantize_then_pack(cuda, n, k, dtype):
             assert torch.equal(got, want) and torch.equal(s, ws)
 
 
+# Rows read twice: odd and even numbers of 512-column chunks around the groups
+# of four and the passes of two, a partial last tile, unaligned rows.
+@pytest.mark.gpu
+@pytest.mark.parametrize("k", [11776, 12288, 12296, 13312, 14336, 14400, 20000, 13825, 14335])
+@pytest.mark.parametrize("dtype", DTYPES, ids=str)
+def test_long_rows_equal_quantize_then_pack(cuda, k, dtype):
+    from nanopointllm_amd import w8a8
+
+    note(f"quant_pack long rows k={k} {dtype}")
+    w = weight(50, k, dtype, k, cuda)
+    w[:, k - 1] = 3.0   # the last column holds the scales
+    for layout in (_lib.ROWS_AS_IS, _lib.ROWS_INTERLEAVE_HALVES):
+        want, ws = two_kernels(w, layout)
+        for parts in ([w], [w[:25], w[25:]]):
+            got, s = w8a8.quant_pack_rows(parts, layout)
+            assert torch.equal(got, want) and torch.equal(s, ws)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,k,dtype,parts,one", [
+    (2048, 11264, torch.float16, 1, True), (2048, 11272, torch.bfloat16, 1, False),
+    (2048, 11272, torch.bfloat16, 2, True), (1040, 16384, torch.float16, 1, False),
+    (1040, 16392, torch.float16, 1, True), (1024, 16392, torch.float16, 1, False),
+    (1024, 16392, torch.float16, 2, False), (64, 4096, torch.float32, 1, True),
+    (2048, 4104, torch.float32, 1, False), (2048, 4104, torch.float32, 2, True),
+    (2, 1 << 28, torch.bfloat16, 1, False)])
+def test_one_kernel_or_two(cuda, monkeypatch, n, k, dtype, parts, one):
+    """The rule that keeps quantizing and packing apart, at its edges, and at a
+    width that the one kernel refuses; the same bytes either way."""
+    from nanopointllm_amd import w8a8
+    from nanopointllm_amd.linear import PackedW8A8Weight
+
+    note(f"quant_pack route {n}x{k} {dtype} in {parts}")
+    calls = []
+    kernel = w8a8.quant_pack_rows
+    monkeypatch.setattr(w8a8, "quant_pack_rows", lambda *a: calls.append(1) or kernel(*a))
+    w = torch.empty((n, k), dtype=dtype, device=cuda)
+    w.normal_(generator=torch.Generator(device=cuda).manual_seed(k))
+    got = PackedW8A8Weight.from_parts(list(w.chunk(parts)))
+    assert bool(calls) == one
+    want, s = two_kernels(w, _lib.ROWS_AS_IS)
+    assert torch.equal(got.packed, want) and torch.equal(got.scale, s)
+
+
 @pytest.mark.gpu
 def test_strided_unaligned_and_non_finite_rows(cuda):
     from nanopointllm_amd import w8a8
