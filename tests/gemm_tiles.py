@@ -35,3 +35,13 @@ def gemm_config(m: int, n: int, cus: int = 256) -> str:
     if code < 0:
         raise ValueError(f"no GEMM tile for {m} x {n}")
     return _lib.GEMM_TILE_NAMES[code]
+
+
+def launched_tile(m: int, n: int, k: int, cus: int = 256) -> str:
+    """The tile an m x n x k product in the GEMM regime runs on:
+    ``pipe-<tile>`` where the pipelined rule (``w8a8_gemm_pipe_config``, asked
+    first by ``launch_gemm``) takes one, else :func:`gemm_config`'s."""
+    from nanopointllm_amd import _lib
+
+    code = _lib.load().w8a8_gemm_pipe_config(m, n, k, cus)
+    return f"pipe-{_lib.GEMM_PIPE_NAMES[code]}" if code >= 0 else gemm_config(m, n, cus)

@@ -4,7 +4,9 @@ k-blocks, two workgroups per CU) when they fill one round on at least half
 the CUs; else one-wave 32x32 tiles with stages of four k-blocks (256 K) when
 there is at most one 64x64 tile per CU, else the 64x64 tile with stages of
 four k-blocks when its tiles fit in two per CU, else the 128x128 tile with
-stages of two k-blocks (128 K) and one workgroup per CU.
+stages of two k-blocks (128 K) and one workgroup per CU.  Products of more than
+15 k-blocks whose tiles would fill three fifths of the CUs run on the pipelined
+tiles instead; the shapes here that do name the one they take.
 
 Bars as for every GEMM path: int32 accumulators bit-exact against the
 oracle's integer product; binary16 / bfloat16 dequant outputs bit-equal to the
@@ -23,7 +25,7 @@ import numpy as np
 import pytest
 import torch
 
-from gemm_tiles import gemm_config as _config
+from gemm_tiles import launched_tile as _config
 from oracle import w8a8_oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -52,18 +54,25 @@ def _case(m, n, k, seed):
     return xq, wq, sx, sw, bias
 
 
-# (m, n, k, config).  K-blocks of 64: 4197 -> 66, 1000 -> 16, 70 -> 2,
-# 3100 -> 49 (a last 128-K stage of one k-block), 4250 -> 67 (a last 256-K
-# stage of three), 11008 -> 172, and 70 (one 256-K stage of two).
+# (m, n, k, config).  K-blocks of 64: 4197 -> 66, 960 and 930 -> 15 (a last
+# 128-K stage of one k-block, a last 256-K stage of three), 700 -> 11, 70 -> 2
+# (one 256-K stage of two), 3100 -> 49, 4250 -> 67, 11008 -> 172.
 SHAPES = [
-    (760, 4096, 4197, "big-deep"),
-    (800, 4100, 3100, "big-deep"),
+    (760, 4096, 960, "big-deep"),
+    (800, 4100, 700, "big-deep"),
     (800, 4096, 70, "big-deep"),
-    (1000, 4096, 1000, "big-deep"),
+    (1000, 4096, 830, "big-deep"),
     (700, 4100, 70, "big-deep"),
-    (130, 12288, 3100, "big-deep"),
-    (300, 6000, 11008, "small-deep"),
-    (300, 6000, 4250, "small-deep"),
+    (130, 12288, 930, "big-deep"),
+    (300, 6000, 960, "small-deep"),
+    (300, 6000, 650, "small-deep"),
+    (256, 4096, 930, "mid"),
+    (760, 4096, 4197, "pipe-128x128"),
+    (800, 4100, 3100, "pipe-128x128"),
+    (1000, 4096, 1000, "pipe-128x128"),
+    (130, 12288, 3100, "pipe-128x96"),
+    (300, 6000, 11008, "pipe-128x96"),
+    (300, 6000, 4250, "pipe-128x96"),
     (100, 1000, 4250, "tiny-deep"),
     (64, 12288, 4250, "tiny-deep"),
     (48, 9000, 70, "tiny-deep"),
@@ -71,7 +80,7 @@ SHAPES = [
     (128, 4096, 11008, "mid"),
     (96, 4100, 4197, "mid"),
     (200, 2048, 3100, "mid"),
-    (256, 4096, 4250, "mid"),
+    (256, 4096, 4250, "pipe-64x64"),
 ]
 
 
@@ -79,7 +88,7 @@ SHAPES = [
 def test_deep_stage_int32_and_dequant(cuda, m, n, k, cfg):
     from nanopointllm_amd import _lib, w8a8
 
-    assert _config(m, n) == cfg
+    assert _config(m, n, k) == cfg
     xq, wq, sx, sw, bias = _case(m, n, k, seed=m + n + k)
     note(f"gemm {cfg} m={m} n={n} k={k}")
     xd, wp = xq.to(cuda), w8a8.pack_rows(wq.to(cuda))
@@ -104,13 +113,13 @@ def test_deep_stage_int32_and_dequant(cuda, m, n, k, cfg):
     np.testing.assert_array_equal(got.cpu().numpy(), want)
 
 
-@pytest.mark.parametrize("m,inter,k", [(760, 2048, 4197), (300, 3000, 4250), (100, 500, 4250),
-                                      (96, 2048, 4197)])
-def test_deep_stage_silu_mul_and_int8_chain(cuda, m, inter, k):
+@pytest.mark.parametrize("m,inter,k,cfg", [
+    (760, 2048, 960, "big-deep"), (300, 3000, 930, "small-deep"), (100, 500, 4250, "tiny-deep"),
+    (96, 2048, 4197, "mid"), (760, 2048, 4197, "pipe-128x128"), (300, 3000, 4250, "pipe-128x96")])
+def test_deep_stage_silu_mul_and_int8_chain(cuda, m, inter, k, cfg):
     from nanopointllm_amd import _lib, w8a8
 
-    cfg = _config(m, 2 * inter)
-    assert cfg in ("big-deep", "small-deep", "tiny-deep", "mid")
+    assert _config(m, 2 * inter, k) == cfg
     xq, wq, sx, sw, _ = _case(m, 2 * inter, k, seed=7 + k)
     note(f"gemm {cfg} silu m={m} inter={inter} k={k}")
     wp = w8a8.pack_rows(wq.to(cuda), _lib.ROWS_INTERLEAVE_HALVES)
@@ -131,12 +140,13 @@ def test_deep_stage_silu_mul_and_int8_chain(cuda, m, inter, k):
     np.testing.assert_array_equal(hq.cpu().numpy(), eq)
 
 
-@pytest.mark.parametrize("m,n,k", [(760, 4096, 4197), (300, 6000, 4250), (100, 1000, 4250),
-                                   (128, 4096, 3100)])
-def test_deep_stage_requant1_epilogue(cuda, m, n, k):
+@pytest.mark.parametrize("m,n,k,cfg", [
+    (760, 4096, 960, "big-deep"), (300, 6000, 930, "small-deep"), (100, 1000, 4250, "tiny-deep"),
+    (128, 4096, 3100, "mid"), (760, 4096, 4197, "pipe-128x128"), (300, 6000, 4250, "pipe-128x96")])
+def test_deep_stage_requant1_epilogue(cuda, m, n, k, cfg):
     from nanopointllm_amd import integer_epilogues as E, w8a8
 
-    assert _config(m, n) in ("big-deep", "small-deep", "tiny-deep", "mid")
+    assert _config(m, n, k) == cfg
     xq, wq, _, sw, _ = _case(m, n, k, seed=5 + k)
     comp = [O.compile_fp16_requant_scale(0.02, float(w), 0.5) for w in sw]
     mult = np.array([c[0] for c in comp], np.uint32)

@@ -1,8 +1,8 @@
 """The narrow GEMM tiles (csrc/gemm.hip ``gemm_kernel``): 112 x 96 (14
 wavefronts of 16 x 48, a 3-stage ring of three k-blocks) and 128 x 96 (8
 wavefronts of 32 x 48, a 2-stage ring of four k-blocks), taken when one round
-of them fills the CUs, as for the O and down projections at M ~ 465..640
-(paged_attention.py:1376, 1488; lightweight_runner.py:362-379).
+of them fills the CUs and K has at most 15 k-blocks of 64 (longer products run
+on the pipelined tiles, and the shapes here that do name the one they take).
 
 Bars as for every GEMM path: int32 accumulators bit-exact against the
 oracle's integer product; dequant outputs bit-equal to the oracle's binary32
@@ -20,7 +20,7 @@ import numpy as np
 import pytest
 import torch
 
-from gemm_tiles import gemm_config
+from gemm_tiles import launched_tile
 from oracle import w8a8_oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -44,10 +44,13 @@ def _case(m, n, k, seed):
 
 SHAPES = [
     # (m, n, k, tile): ragged rows / columns, K from one k-block to 11008
-    (560, 4096, 4096, "t112x96"), (560, 4096, 11008, "t112x96"), (470, 3900, 1000, "t112x96"),
+    (560, 4096, 960, "t112x96"), (560, 4096, 700, "t112x96"), (470, 3900, 900, "t112x96"),
     (500, 4090, 64, "t112x96"), (545, 4000, 130, "t112x96"),
-    (567, 4096, 4096, "t128x96"), (640, 4090, 11008, "t128x96"), (600, 4096, 130, "t128x96"),
-    (620, 4096, 64, "t128x96"), (580, 3950, 1111, "t112x96"),
+    (567, 4096, 960, "t128x96"), (640, 4090, 830, "t128x96"), (600, 4096, 130, "t128x96"),
+    (620, 4096, 64, "t128x96"), (580, 3950, 600, "t112x96"),
+    (560, 4096, 4096, "pipe-128x96"), (560, 4096, 11008, "pipe-128x96"),
+    (470, 3900, 1000, "pipe-128x64"), (567, 4096, 4096, "pipe-128x96"),
+    (640, 4090, 11008, "pipe-128x96"), (580, 3950, 1111, "pipe-128x96"),
 ]
 
 
@@ -55,7 +58,7 @@ SHAPES = [
 def test_narrow_int32_and_dequant(cuda, m, n, k, cfg):
     from nanopointllm_amd import w8a8
 
-    assert gemm_config(m, n) == cfg
+    assert launched_tile(m, n, k) == cfg
     xq, wq, sx, sw, bias = _case(m, n, k, seed=m + n + k)
     note(f"gemm {cfg} m={m} n={n} k={k}")
     xd, wp = xq.to(cuda), w8a8.pack_rows(wq.to(cuda))
@@ -74,13 +77,15 @@ def test_narrow_int32_and_dequant(cuda, m, n, k, cfg):
             np.testing.assert_array_equal(got, want, err_msg=f"{dt} bias={b is not None}")
 
 
-@pytest.mark.parametrize("m,inter,k,cfg", [(560, 2048, 4096, "t112x96"), (500, 2000, 333, "t112x96"),
-                                            (567, 2048, 1000, "t128x96"), (630, 2048, 640, "t128x96")])
+@pytest.mark.parametrize("m,inter,k,cfg", [(560, 2048, 960, "t112x96"), (500, 2000, 333, "t112x96"),
+                                            (567, 2048, 900, "t128x96"), (630, 2048, 640, "t128x96"),
+                                            (560, 2048, 4096, "pipe-128x96"),
+                                            (567, 2048, 1000, "pipe-128x96")])
 def test_narrow_silu_mul_int8_chain_and_two_phase(cuda, m, inter, k, cfg):
     from nanopointllm_amd import _lib, w8a8
 
     n = 2 * inter
-    assert gemm_config(m, n) == cfg
+    assert launched_tile(m, n, k) == cfg
     xq, wq, sx, sw, _ = _case(m, n, k, seed=11 + k)
     note(f"gemm {cfg} silu m={m} inter={inter} k={k}")
     wp = w8a8.pack_rows(wq.to(cuda), _lib.ROWS_INTERLEAVE_HALVES)
@@ -106,13 +111,15 @@ def test_narrow_silu_mul_int8_chain_and_two_phase(cuda, m, inter, k, cfg):
     np.testing.assert_array_equal(out.scale.cpu().numpy(), ts[:, 0])
 
 
-@pytest.mark.parametrize("m,n,k,cfg", [(560, 4096, 1000, "t112x96"), (600, 4096, 2000, "t128x96")])
+@pytest.mark.parametrize("m,n,k,cfg", [(560, 4096, 900, "t112x96"), (600, 4096, 960, "t128x96"),
+                                       (560, 4096, 1000, "pipe-128x96"),
+                                       (600, 4096, 2000, "pipe-128x96")])
 def test_narrow_integer_epilogues(cuda, m, n, k, cfg):
     """requant1 (multiplier / shift int8 out) and the single-rounding
     int32 -> bf16 dequant on the narrow tiles."""
     from nanopointllm_amd import _lib, integer_epilogues as E, w8a8
 
-    assert gemm_config(m, n) == cfg
+    assert launched_tile(m, n, k) == cfg
     xq, wq, sx, sw, _ = _case(m, n, k, seed=5 + k)
     comp = [O.compile_fp16_requant_scale(0.02, float(w), 0.5) for w in sw]
     mult = np.array([c[0] for c in comp], np.uint32)

@@ -1,9 +1,9 @@
-"""The pipelined GEMM tiles (csrc/gemm.hip ``gemm_pipe_kernel``), one shape per
-tile that the library's own rule gives to it: ragged in M and N (partial
-tiles, a partial last 16-row block), K of 17 to 20 k-blocks with a partial last
-one (every remainder of the unrolled loop).  int32 products exact, the float
-epilogues bit-equal to the oracle's, the integer ones exact; and the rule
-itself (no GPU)."""
+"""The pipelined GEMM tiles (csrc/gemm_pipe.hip ``gemm_pipe_kernel``), one
+shape per tile that the library's own rule gives to it: ragged in M and N
+(partial tiles, a partial last 16-row block), K with a partial last k-block,
+and every remainder of each tile's unrolled loop (six k-blocks for the 352-wide
+tiles, two for the others).  int32 products exact, the float epilogues bit-equal
+to the oracle's, the integer ones exact; and the rule itself (no GPU)."""
 from __future__ import annotations
 
 import sys
@@ -12,7 +12,7 @@ import numpy as np
 import pytest
 import torch
 
-from gemm_tiles import gemm_config
+from gemm_tiles import launched_tile
 from oracle import w8a8_oracle as O
 
 SHAPES = [(66, 4886, 1030, "64x64"), (65, 9858, 1100, "128x64"), (129, 8230, 1160, "128x96"),
@@ -20,6 +20,11 @@ SHAPES = [(66, 4886, 1030, "64x64"), (65, 9858, 1100, "128x64"), (129, 8230, 116
           (195, 20588, 1160, "256x128"), (260, 21950, 1250, "256x192"),
           (515, 16350, 1030, "192x288"), (580, 18510, 1100, "256x256"),
           (577, 21800, 1160, "192x352"), (580, 22570, 1250, "256x352")]
+# 16 to 21 k-blocks: what the unrolled loop of six leaves is 4, 5, 0, 1, 2, 3.
+SIX_KS = (1000, 1030, 1100, 1160, 1250, 1340)
+# Every remainder of each tile's unrolled loop.
+REMAINDERS = [(m, n, k, t) for m, n, _, t in SHAPES
+              for k in (SIX_KS if t in ("192x352", "256x352") else (1030, 1100))]
 # One shape per tile of the ring kernels, at a K that leaves it to them.
 RING = [(100, 1000, 900, "tiny-deep"), (300, 6000, 900, "small-deep"), (760, 4096, 900, "big-deep"),
         (567, 12288, 300, "big"), (128, 4096, 900, "mid"), (560, 12288, 300, "wd7x2"),
@@ -43,6 +48,9 @@ def pipe_config(m, n, k, cus=256):
     (1024, 22016, 4096, "256x352"), (2048, 4096, 4096, "256x128"), (2048, 12288, 4096, "256x192"),
     (201, 12288, 4096, "128x96"), (201, 4096, 4096, "64x64"), (448, 4096, 4096, "128x64"),
     (768, 22016, 4096, "192x352"), (100, 4096, 11008, None), (64, 22016, 8192, None), (2048, 12288, 960, None),
+    # fewer than 16 k-blocks of 64 stay on the ring tiles
+    (560, 4096, 960, None), (560, 4096, 961, "128x96"), (560, 4096, 1023, "128x96"),
+    (500, 12000, 1000, "192x160"),
     (0, 4096, 4096, None), (560, 4096, 0, None)])
 def test_rule(m, n, k, tile):
     assert pipe_config(m, n, k) == tile
@@ -65,10 +73,7 @@ def _case(m, n, k, dev):
 def test_tile_int32_and_dequant(cuda, m, n, k, tile):
     from nanopointllm_amd import w8a8
 
-    if k < 1024:
-        assert pipe_config(m, n, k) is None and gemm_config(m, n) == tile
-    else:
-        assert pipe_config(m, n, k) == tile
+    assert launched_tile(m, n, k) == (tile if k <= 960 else f"pipe-{tile}")
     note(f"gemm {tile} m={m} n={n} k={k}")
     xq, wq, eacc, sx, sw, bias = _case(m, n, k, cuda)
     wp = w8a8.pack_rows(wq)
@@ -79,6 +84,20 @@ def test_tile_int32_and_dequant(cuda, m, n, k, tile):
         exp = torch.from_numpy(O.dequant_epilogue(eacc, sx, sw, None if b is None else bias))
         np.testing.assert_array_equal(y.float().cpu().numpy(), exp.to(dt).float().numpy(),
                                       err_msg=str(dt))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k,tile", REMAINDERS)
+def test_every_remainder_of_the_unrolled_loop(cuda, m, n, k, tile):
+    from nanopointllm_amd import w8a8
+
+    assert pipe_config(m, n, k) == tile
+    note(f"gemm pipe remainder {tile} m={m} n={n} k={k}")
+    g = torch.Generator(device=cuda).manual_seed(k)
+    xq = torch.randint(-127, 128, (m, k), generator=g, dtype=torch.int8, device=cuda)
+    wq = torch.randint(-127, 128, (n, k), generator=g, dtype=torch.int8, device=cuda)
+    want = torch.matmul(xq.double(), wq.double().T).to(torch.int32)
+    assert torch.equal(w8a8.gemm_i32(xq, w8a8.pack_rows(wq), n), want)
 
 
 @pytest.mark.gpu

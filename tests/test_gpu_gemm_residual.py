@@ -83,9 +83,12 @@ def test_layer_bits_do_not_depend_on_the_route(cuda, rows):
     runner = W8A8LlamaRunner(model, lambda q, k, v, i, state: q.reshape(q.shape[0], -1))
     mod = runner.layers[0]
     x = torch.randn(rows, h, generator=g, device=cuda).half()
+    route = lambda: mod._adds_in_epilogues(x, x)  # noqa: E731
+    assert route() == (rows > 64)
     out = mod(x)
     seen = []
     handle = mod.o_proj.register_forward_hook(lambda m, a, y: seen.append(tuple(y.shape)))
+    assert not route()
     hooked = mod(x)
     handle.remove()
     assert seen == [(rows, h)]

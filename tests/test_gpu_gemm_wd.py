@@ -1,8 +1,9 @@
 """The weights-direct GEMM tile (csrc/gemm.hip ``gemm_wd_kernel``): 112 x 256
-(8 wavefronts of 112 x 32), taken when one round of it fills the CUs, as for
-the packed QKV projection at M ~ 560 (paged_attention.py:1349-1352;
-lightweight_runner.py:389-404).  Weight fragments go straight from memory into
-registers several k-blocks ahead; only the activations pass through LDS.
+(8 wavefronts of 112 x 32), taken when one round of it fills the CUs and K has
+at most 15 k-blocks of 64 (longer products run on the pipelined tiles, and the
+shapes here that do name the one they take).  Weight fragments go straight from
+memory into registers several k-blocks ahead; only the activations pass through
+LDS.
 
 Bars as for every GEMM path: int32 accumulators bit-exact against the
 oracle's integer product; dequant outputs bit-equal to the oracle's binary32
@@ -10,7 +11,8 @@ result rounded once; SiLU*mul equal to the oracle's; the int8 requant of h
 and the integer requant (requant1) bit-exact; the two-phase per-block maxima
 giving hq and scales bit-exact against the per-token quantization of h.
 Shapes are ragged in M, N and K, including K of one or a few k-blocks (fewer
-than the prefetch depth) and K that leaves a partial unrolled loop.
+than the prefetch depth), of 11 to 15 (the unrolled loop of 10 and what is left
+behind it) and K that leaves a partial one.
 """
 from __future__ import annotations
 
@@ -20,7 +22,7 @@ import numpy as np
 import pytest
 import torch
 
-from gemm_tiles import gemm_config
+from gemm_tiles import launched_tile
 from oracle import w8a8_oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -44,9 +46,11 @@ def _case(m, n, k, seed):
 
 SHAPES = [
     # (m, n, k, tile): ragged rows / columns, K from one k-block to 11008
-    (560, 12288, 4096, "wd7x2"), (500, 12000, 1000, "wd7x2"), (545, 12100, 64, "wd7x2"),
-    (480, 12288, 200, "wd7x2"), (555, 11900, 2700, "wd7x2"),
-    (400, 16000, 1111, "wd7x2"), (470, 11100, 64, "wd7x2"), (465, 13000, 130, "wd7x2"),
+    (560, 12288, 960, "wd7x2"), (500, 12000, 641, "wd7x2"), (545, 12100, 64, "wd7x2"),
+    (480, 12288, 200, "wd7x2"), (555, 11900, 700, "wd7x2"), (480, 12100, 640, "wd7x2"),
+    (400, 16000, 800, "wd7x2"), (470, 11100, 64, "wd7x2"), (465, 13000, 130, "wd7x2"),
+    (560, 12288, 4096, "pipe-192x160"), (500, 12000, 1000, "pipe-192x160"),
+    (555, 11900, 2700, "pipe-192x160"), (400, 16000, 1111, "pipe-256x128"),
 ]
 
 
@@ -54,7 +58,7 @@ SHAPES = [
 def test_wd_int32_and_dequant(cuda, m, n, k, cfg):
     from nanopointllm_amd import w8a8
 
-    assert gemm_config(m, n) == cfg
+    assert launched_tile(m, n, k) == cfg
     xq, wq, sx, sw, bias = _case(m, n, k, seed=m + n + k)
     note(f"gemm {cfg} m={m} n={n} k={k}")
     xd, wp = xq.to(cuda), w8a8.pack_rows(wq.to(cuda))
@@ -73,13 +77,15 @@ def test_wd_int32_and_dequant(cuda, m, n, k, cfg):
             np.testing.assert_array_equal(got, want, err_msg=f"{dt} bias={b is not None}")
 
 
-@pytest.mark.parametrize("m,inter,k,cfg", [(520, 6100, 4096, "wd7x2"), (560, 6144, 333, "wd7x2"),
-                                            (470, 6000, 1000, "wd7x2"), (400, 7500, 640, "wd7x2")])
+@pytest.mark.parametrize("m,inter,k,cfg", [(520, 6100, 960, "wd7x2"), (560, 6144, 333, "wd7x2"),
+                                            (470, 6000, 730, "wd7x2"), (400, 7500, 640, "wd7x2"),
+                                            (520, 6100, 4096, "pipe-192x160"),
+                                            (470, 6000, 1000, "pipe-192x160")])
 def test_wd_silu_mul_int8_chain_and_two_phase(cuda, m, inter, k, cfg):
     from nanopointllm_amd import _lib, w8a8
 
     n = 2 * inter
-    assert gemm_config(m, n) == cfg
+    assert launched_tile(m, n, k) == cfg
     xq, wq, sx, sw, _ = _case(m, n, k, seed=11 + k)
     note(f"gemm {cfg} silu m={m} inter={inter} k={k}")
     wp = w8a8.pack_rows(wq.to(cuda), _lib.ROWS_INTERLEAVE_HALVES)
@@ -105,13 +111,15 @@ def test_wd_silu_mul_int8_chain_and_two_phase(cuda, m, inter, k, cfg):
     np.testing.assert_array_equal(out.scale.cpu().numpy(), ts[:, 0])
 
 
-@pytest.mark.parametrize("m,n,k,cfg", [(560, 12288, 1000, "wd7x2"), (400, 15000, 2000, "wd7x2")])
+@pytest.mark.parametrize("m,n,k,cfg", [(560, 12288, 700, "wd7x2"), (400, 15000, 960, "wd7x2"),
+                                       (560, 12288, 1000, "pipe-192x160"),
+                                       (400, 15000, 2000, "pipe-256x128")])
 def test_wd_integer_epilogues(cuda, m, n, k, cfg):
     """requant1 (multiplier / shift int8 out) and the single-rounding
     int32 -> bf16 dequant on the weights-direct tiles."""
     from nanopointllm_amd import _lib, integer_epilogues as E, w8a8
 
-    assert gemm_config(m, n) == cfg
+    assert launched_tile(m, n, k) == cfg
     xq, wq, sx, sw, _ = _case(m, n, k, seed=5 + k)
     comp = [O.compile_fp16_requant_scale(0.02, float(w), 0.5) for w in sw]
     mult = np.array([c[0] for c in comp], np.uint32)
@@ -150,7 +158,7 @@ def test_linear_packed_equals_linear_i8in(cuda, m, n, k, epi):
 
     xq, wq, sx, sw, bias = _case(m, n, k, seed=31 + m)
     layout = _lib.ROWS_INTERLEAVE_HALVES if epi == "silu" else _lib.ROWS_AS_IS
-    note(f"linear_packed m={m} n={n} k={k} {epi} tile={gemm_config(m, n)}")
+    note(f"linear_packed m={m} n={n} k={k} {epi} tile={launched_tile(m, n, k)}")
     xd, wp = xq.to(cuda), w8a8.pack_rows(wq.to(cuda), layout)
     sxt, swt, bt = (torch.from_numpy(a).to(cuda) for a in (sx, sw, bias))
     code = {"i32": _lib.EPI_I32, "silu": _lib.EPI_SILU_MUL}.get(epi, _lib.EPI_DEQUANT)

@@ -2,7 +2,8 @@
 128-row tiles of 192, 224 or 256 columns (8 waves each, three LDS stages):
 the widest whose tiles still fit in one round of workgroup slots, else (for
 several rounds) 128x256, or from two full rounds of them the 256x256 tile
-(16 waves, one workgroup per CU).
+(16 waves, one workgroup per CU).  At most 15 k-blocks of 64: longer products
+run on the pipelined tiles.
 
 Bars as for every GEMM path: int32 accumulators bit-exact against the
 oracle's integer product; binary16 / bfloat16 / binary32 dequant outputs
@@ -21,7 +22,7 @@ import numpy as np
 import pytest
 import torch
 
-from gemm_tiles import gemm_config
+from gemm_tiles import launched_tile
 from oracle import w8a8_oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -56,7 +57,7 @@ def _case(m, n, k, seed):
 def test_wide_tile_int32_and_dequant(cuda, m, n, k, cfg):
     from nanopointllm_amd import w8a8
 
-    assert gemm_config(m, n) == cfg
+    assert launched_tile(m, n, k) == cfg
     xq, wq, sx, sw, bias = _case(m, n, k, seed=m + n + k)
     note(f"gemm {cfg} m={m} n={n} k={k}")
     xd, wp = xq.to(cuda), w8a8.pack_rows(wq.to(cuda))
@@ -80,7 +81,7 @@ def test_wide_tile_int32_and_dequant(cuda, m, n, k, cfg):
 def test_wide_tile_silu_mul_and_int8_chain(cuda, m, inter, k, cfg):
     from nanopointllm_amd import _lib, w8a8
 
-    assert gemm_config(m, 2 * inter) == cfg
+    assert launched_tile(m, 2 * inter, k) == cfg
     xq, wq, sx, sw, _ = _case(m, 2 * inter, k, seed=11 + k)
     note(f"gemm {cfg} silu m={m} inter={inter} k={k}")
     wp = w8a8.pack_rows(wq.to(cuda), _lib.ROWS_INTERLEAVE_HALVES)
@@ -109,7 +110,7 @@ def test_requant1_epilogue_at_a_wide_shape(cuda, m, n, k, cfg):
     oracle elsewhere), and a random sample of entries against the oracle."""
     from nanopointllm_amd import integer_epilogues as E, w8a8
 
-    assert gemm_config(m, n) == cfg
+    assert launched_tile(m, n, k) == cfg
     xq, wq, _, sw, _ = _case(m, n, k, seed=5)
     comp = [O.compile_fp16_requant_scale(0.02, float(w), 0.5) for w in sw]
     mult = np.array([c[0] for c in comp], np.uint32)

@@ -176,10 +176,10 @@ def down_full(cuda):
 
 
 def test_full_size_tiles_are_covered():
-    from gemm_tiles import gemm_config
+    from gemm_tiles import launched_tile
 
-    tiles = {gemm_config(m, 22016) for m in FULL_M}
-    assert len(tiles) >= 4, tiles
+    tiles = {launched_tile(m, 22016, 4096) for m in FULL_M}
+    assert tiles == {"pipe-192x288", "pipe-192x352", "pipe-256x352"}
 
 
 @pytest.mark.parametrize("m", FULL_M)
@@ -187,13 +187,13 @@ def test_two_phase_full_size_gateup(cuda, gateup_full, down_full, m):
     """h equals the plain SiLU*mul linear, hq and its scales are bit-exact
     against the oracle's per-token quantization of that h, and the down
     projection on hq is exact against the oracle (on a sample of rows)."""
-    from gemm_tiles import gemm_config
+    from gemm_tiles import launched_tile
     from nanopointllm_amd import _lib, w8a8
     import workloads as W
 
     p = gateup_full
     x = W.prefill_activations(m, 4096, seed=m, point_tokens=min(513, m - 7)).to(cuda)
-    note(f"two-phase full size m={m} tile={gemm_config(m, 22016)}")
+    note(f"two-phase full size m={m} tile={launched_tile(m, 22016, 4096)}")
     plain = w8a8.linear_dynamic(x, p.packed, p.scale, p.bias, p.out_features,
                                 epilogue=_lib.EPI_SILU_MUL)
     out = w8a8.gateup_silu_mul_two_phase(x, p.packed, p.scale, p.bias, p.out_features)
