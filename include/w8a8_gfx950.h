@@ -113,9 +113,9 @@ int64_t w8a8_workspace_bytes(int64_t m, int64_t k);
  * product in the GEMM regime on a device with `cus` compute units: 0 =
  * 128x128, 1 = 192x160, 2 = 256x128, 3 = 256x192, 4 = 192x288, 5 = 256x256,
  * 6 = 256x352, 7 = 128x96, 8 = 128x64, 9 = 64x64 (4 wavefronts), 10 =
- * 192x352; -1 where none is taken (K below 1024, at most 64 rows, too few
- * tiles for the CUs, or a size not positive) and the tile of
- * w8a8_gemm_tile_config is.  A pure function of its arguments. */
+ * 192x352; -1 where none is taken (K of at most 960, that is fewer than 16
+ * k-blocks of 64; at most 64 rows; too few tiles for the CUs; or a size not
+ * positive) and the tile of w8a8_gemm_tile_config is.  A pure function of its arguments. */
 int w8a8_gemm_pipe_config(int64_t m, int64_t n, int64_t k, int64_t cus);
 
 /* GEMM workgroup tile that w8a8_gemm_i32 / w8a8_linear / w8a8_linear_i8in

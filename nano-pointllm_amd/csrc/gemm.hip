@@ -5,8 +5,12 @@
 // 1488; llama/lightweight_runner.py:320-404) for the int8 contract of
 // integer_linear_per_output_reference (nanopointllm/compression/w8a8.py:118-139).
 //
-// These kernels take what gemm_pipe_choice (gemm_pipe.hip) leaves: K below 1024,
-// and products whose tiles there would not fill three fifths of the CUs.
+// These kernels take what gemm_pipe_choice (gemm_pipe.hip) leaves: products of
+// fewer than 16 k-blocks (K <= 960), at most 64 rows, and those whose tiles
+// there would not fill three fifths of the CUs.  The last two take only the
+// 32x32, 64x32, 64x64 and two-per-CU 128x128 tiles; the others below (112x256
+// weights-direct, 112x96, 128x96, 128x192, 128x224, 128x256, 256x256 and 128x128
+// with one per CU) serve K <= 960 alone.
 //
 // Design (MFMA-bound), chosen by measurement on MI355X (gemm_kernel; the
 // weights-direct gemm_wd_kernel further below keeps the weights out of LDS):
@@ -326,14 +330,16 @@ hipError_t launch_cfg(GemmParams p, hipStream_t st) {
   return hipGetLastError();
 }
 
-// Tile configurations, chosen by tile count (figures of longer K are from before
-// the pipelined tiles took those products; measured on MI355X, random data,
-// cold weights, LLaMA-7B projections at M = 256..2048).  A launch is fastest
+// Tile configurations, chosen by tile count.  Measured on MI355X, random data,
+// cold weights, LLaMA-7B projections (K = 4096 and 11008) at M = 256..2048,
+// which the pipelined tiles have since taken from all but the 32x32, 64x32, 64x64
+// and two-per-CU 128x128 ones: the figures below order the ring tiles among
+// themselves, and the projections named are no longer what they run.  A launch is fastest
 // when its tiles fill one round of workgroup slots (2 per CU) as closely as
 // possible, and when several rounds are needed, with the widest tile:
 //   * first the one-workgroup-per-CU tiles taken when one round of them fills
-//     the CUs (gemm_tile_choice): 112x256 weights-direct (gemm_wd_kernel,
-//     packed QKV at M = 449..560), then 112x96 and 128x96 (O and down at
+//     the CUs (gemm_tile_choice): 112x256 weights-direct (gemm_wd_kernel;
+//     N = 12288 at M = 449..560), then 112x96 and 128x96 (N = 4096 at
 //     M = 465..640);
 //   * past 64 rows (M > 64), 64x32 tiles (4 waves of 32x16, a 3-stage ring of
 //     four k-blocks, 2 workgroups per CU) when they fit in one round and
@@ -354,8 +360,8 @@ hipError_t launch_cfg(GemmParams p, hipStream_t st) {
 //     9-13% faster on QKV at M = 64;
 //   * else the widest of 128x192, 128x224 and 128x256 whose tiles still fit
 //     in one round, trying the narrowest first (8 waves of 32x96, 32x112 or
-//     64x64, 3-stage ring): 128x224 takes gate/up at M = 560 in 495 tiles,
-//     8% faster than 430 tiles of 128x256;
+//     64x64, 3-stage ring): N = 22016 at M = 560 in 495 tiles of 128x224 was
+//     8% faster than in 430 of 128x256;
 //   * else (several rounds) 128x256, except just past one round of those
 //     (1 to 1.25 tiles per slot), where the few tiles of the second round cost
 //     more than the wider tile saves and 128x128 is kept, and except from two
@@ -406,10 +412,10 @@ struct RingLaunch {
 int gemm_tile_choice(int64_t MB, int64_t NB, int64_t cus) {
   // The 112 x 256 weights-direct tile when one round of it (one workgroup per
   // CU) fills at least 85% of the CUs with at least 85% of the tile rows in
-  // use (the packed QKV at M = 449..560).  A 144 x 64 weights-direct tile for
-  // O and down at the same M measured slower than the 128 x 128 deep ring
-  // (27.2 vs 23.5 us and 59.6 vs 51.3 us with the fp16 epilogue), so those
-  // keep the LDS-ring tiles.
+  // use (N = 12288 at M = 449..560).  A 144 x 64 weights-direct tile for
+  // N = 4096 at the same M measured slower than the 128 x 128 deep ring
+  // (K = 4096 27.2 vs 23.5 us, K = 11008 59.6 vs 51.3 us with the fp16
+  // epilogue), so those keep the LDS-ring tiles.
   if (MB > 4) {
     const int64_t tm = ceil_div(MB, 7);
     const int64_t tiles = tm * ceil_div(NB, 16);
@@ -417,10 +423,10 @@ int gemm_tile_choice(int64_t MB, int64_t NB, int64_t cus) {
   }
   // Narrow tiles (96 columns) when one round of them, at least four tile rows
   // deep, fills at least 80% of the CUs with at least 85% of the tile rows in
-  // use: O and down (N = 4096) at M = 465..640, where 128x128 tiles leave 96
-  // of 256 CUs idle.  Measured at M = 560 (fp16 epilogue): 112x96 takes O in
-  // 20.8 against 23.6 us and down in 48.1 against 58.5 us; at M = 567 (36
-  // row blocks) 128x96 takes O in 21.6 against 23.8 us.  The 14 wavefronts of
+  // use: N = 4096 at M = 465..640, where 128x128 tiles leave 96 of 256 CUs
+  // idle.  Measured at M = 560 (fp16 epilogue, K = 4096 and 11008, before the
+  // pipelined tiles took those): 112x96 20.8 against 23.6 us and 48.1 against
+  // 58.5; at M = 567 (36 row blocks) 128x96 21.6 against 23.8 us.  The 14 wavefronts of
   // 112x96 each own a 16-row strip.
   if (MB > 4) {
     auto one_round = [&](int64_t rows, int64_t cols) {

@@ -1,5 +1,6 @@
 // Prefill-regime W8A8 GEMM on pipelined tiles: the shapes that gemm_pipe_choice
-// gives a tile (K >= 1024, more than 64 rows, tiles for three fifths of the CUs);
+// gives a tile (16 k-blocks or more, so K > 960; more than 64 rows; tiles for
+// three fifths of the CUs);
 // the others stay on gemm.hip's ring kernels.
 //
 // Replaces the prefill/mixed projections (llama/paged_attention.py:1349-1352,
@@ -15,10 +16,11 @@ namespace {
 // wavefront BR x BC 16x16 blocks (tile 16 WM BR x 16 WN BC), an S-slot LDS ring of single
 // k-blocks (64 K) and one barrier per k-block.
 //   * Each wavefront keeps the fragments of its shorter side of a k-block in
-//     registers (`held`, double-buffered) and passes the longer side's through
-//     R registers (`strm`), every fragment read from LDS about a k-block before
-//     its MFMAs, also across the barriers: no MFMA waits for an LDS read
-//     issued behind a barrier.  (gemm_kernel reads a k-block's fragments after
+//     registers (`held`, double-buffered: read up to a k-block before its
+//     MFMAs) and passes the longer side's through R registers (`strm`, read R
+//     fragments ahead: a quarter of a k-block on the 352-wide tiles, a third on
+//     192 x 288, half on 256 x 256, a whole one on the others), also across the
+//     barriers: no MFMA waits for an LDS read issued right behind a barrier.  (gemm_kernel reads a k-block's fragments after
 //     its barrier, so all wavefronts read at once while the matrix pipes idle.)
 //   * The k-loop has no branch: operand copies past the last k-block re-read it
 //     into slots that nothing reads, and wavefronts without a share of their
@@ -211,9 +213,10 @@ struct PipeLaunch {
 // 57 for the ring of 16 wavefronts) and 256x128 at 2048 (34 / 77 against 38 / 99).
 // Taken where the tiles fill three fifths of the CUs; below that the smaller
 // ring tiles cover more of them (down at 100 rows: 27.0 against 28.0 us on 64x64).
-// From K = 1024: filling a ring of up to 16 k-blocks is a large part of a shorter
+// From 16 k-blocks: filling a ring of up to 16 is a large part of a shorter
 // product (2048 x 12288 x 512 21.4 on the ring against 22.0, 560 x 4096 x 768 6.8
-// against 7.0, though 2048 x 22016 x 768 59.8 against 52.0).
+// against 7.0).  One line for all sizes is not the best one: products of several
+// rounds gain earlier (2048 x 22016 x 768 59.8 on the ring against 52.0).
 int gemm_pipe_choice(int64_t MB, int64_t NB, int64_t KB, int64_t cus) {
   struct Tile {
     GemmPipe id;

@@ -337,7 +337,7 @@ __device__ inline void qdq_store8(const QdqOut& o, int64_t row, int64_t k0, int 
 // 8-column chunk each, so a group's scale takes log2(LPG) lane exchanges and
 // the matrix is read and written once.  Bound: HBM (2 bytes in, 3 out per
 // 16-bit weight): 4096 x 11008 bfloat16 in groups of 128 takes 44.5 us, 5.1
-// TB/s, a large copy's rate on this card; a workgroup per group (quantization
+// TB/s (a large copy reaches 4.8, read and written); a workgroup per group (quantization
 // alone 230 us) and torch's elementwise passes behind it took 602.
 template <typename TX, int LPG>
 __global__ __launch_bounds__(kQuantThreads) void qdq_groups_kernel(
