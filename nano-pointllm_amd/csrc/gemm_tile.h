@@ -128,11 +128,13 @@ struct TileScales {
 // packs its four (or with SiLU, whose gate/up pairs are adjacent columns, two)
 // outputs itself.
 //
-// 32-bit outputs leave as 16-byte stores.  16- and 8-bit outputs pass through
-// the operand ring's LDS at `stage` and leave as 16-byte chunks of whole tile
-// rows, in passes of as many row blocks per wavefront as STAGE_BYTES hold.
-// The LDS row stride is an odd multiple of 16 bytes: the 16 rows a wavefront
-// writes at once then start in different banks.
+// The outputs pass through the operand ring's LDS at `stage` and leave as
+// 16-byte chunks of whole tile rows, in passes of as many row blocks per
+// wavefront as STAGE_BYTES hold.  The LDS row stride is an odd multiple of 16
+// bytes: the 16 rows a wavefront writes at once then start in different banks.
+// 32-bit outputs too: stored from the registers, 64 bytes (half a line) of 16
+// rows at a time, int32 calls of 2048 x 22016 x 768 took 103 us, 1024 x 12288 x
+// 512 24.5 and 560 x 12288 x 4096 38.9; through LDS 75.5, 16.9 and 31.6.
 //
 // Bound by VALU work and stores: 12 thousand shader cycles for a 256 x 256
 // binary16 tile of 8 wavefronts, 5.6 for 128 x 256, 25 with SiLU on 256 x 256.
@@ -151,12 +153,11 @@ __device__ inline void store_tile(const GemmParams& p, i32x4 (&acc)[BR][BC], int
   constexpr int OW = kHalfCols ? 2 : 4;                             // outputs per lane and block
   constexpr int BNO = kHalfCols ? BN / 2 : BN;
   constexpr int kOutBytes = static_cast<int>(sizeof(TY));
-  constexpr bool kStage = kOutBytes < 4;
   constexpr int kRowBytes = BNO * kOutBytes;
   constexpr int kStride = (kRowBytes / 16 | 1) * 16;
   static_assert(kRowBytes % 16 == 0, "tile rows are whole 16-byte chunks");
   constexpr int kFit = STAGE_BYTES / (WM * 16 * kStride);
-  constexpr int IPP = !kStage || kFit > BR ? BR : kFit;  // row blocks per wavefront and pass
+  constexpr int IPP = kFit > BR ? BR : kFit;  // row blocks per wavefront and pass
   static_assert(IPP >= 1, "a pass holds at least one row block per wavefront");
 
   const int quad = lane >> 4;
@@ -230,129 +231,107 @@ __device__ inline void store_tile(const GemmParams& p, i32x4 (&acc)[BR][BC], int
 
   const bool vec_ok =
       ((reinterpret_cast<uintptr_t>(p.y) | static_cast<uintptr_t>(p.ldy * kOutBytes)) & 15) == 0;
-  if constexpr (!kStage) {
+  char* const st = static_cast<char*>(stage);
+  constexpr int EV = 16 / kOutBytes;    // outputs per 16-byte chunk
+  constexpr int CPR = kRowBytes / 16;   // chunks per tile row
+  constexpr int NT = WM * WN * 64;
+  constexpr int RPP = NT / CPR;         // rows per sweep; threads past RPP * CPR idle
+  static_assert(RPP >= 1, "a sweep covers at least one tile row");
+  const int64_t n_out_total = kHalfCols ? p.N / 2 : p.N;
+  const int64_t n0_out = kHalfCols ? n0 / 2 : n0;
+  const int crow = static_cast<int>(threadIdx.x) / CPR;
+  const int cchunk = static_cast<int>(threadIdx.x) % CPR;
+  const int64_t nc = n0_out + cchunk * EV;  // this thread's first output column
+  // Output row of tile-local row `row` of the pass over blocks i0 .. i0 + ni.
+  auto out_row = [&](int row, int i0, int ni) {
+    return m0 + 16 * (row / (16 * ni) * BR + i0) + row % (16 * ni);
+  };
+  // Residual add, y = dtype(dtype(dequant) + res); with ROOMY the pass's
+  // residual chunks (up to 8 per thread) are requested before its arithmetic.
+  // It spares O and down of a prefill layer a pass over their rows (three
+  // trips through memory).
+  constexpr bool kRes = EPI == kEpiDequant && kOutBytes == 2;
+  constexpr int kSweeps = (WM * 16 * IPP + RPP - 1) / RPP;
+  constexpr bool kEarly = kRes && ROOMY && kSweeps <= 8;
+  const bool res_vec = kRes && p.res != nullptr && nc + EV <= n_out_total &&
+                       ((reinterpret_cast<uintptr_t>(p.res) |
+                         static_cast<uintptr_t>(p.ld_res * kOutBytes)) & 15) == 0;
+  [[maybe_unused]] Pack<TY, EV> early[kEarly ? kSweeps : 1];
+#pragma unroll
+  for (int i0 = 0; i0 < BR; i0 += IPP) {
+    const int ni = BR - i0 < IPP ? BR - i0 : IPP;  // compile-time after unrolling
+    if constexpr (kEarly) {
+      if (res_vec) {
+#pragma unroll
+        for (int t = 0; t < kSweeps; ++t) {
+          const int row = t * RPP + crow;
+          const int64_t m = out_row(row, i0, ni);
+          const bool ok = crow < RPP && row < WM * 16 * ni && m < p.M;
+          early[t] = *reinterpret_cast<const Pack<TY, EV>*>(
+              static_cast<const TY*>(p.res) + (ok ? m : 0) * p.ld_res + nc);
+        }
+      }
+    }
+    ring_barrier();  // the ring's (or the last pass's) readers are done
 #pragma unroll
     for (int j = 0; j < BC; ++j) {
       const Cols cj = cols_of(j);
 #pragma unroll
-      for (int i = 0; i < BR; ++i) {
-        const int64_t m = m0 + row_of(i);
-        const int64_t n = n0 + col_of(j);
-        const Pack<TY, 4> o = outputs(i, j, cj);
-        if (m < p.M && n < p.N) {
-          TY* const dst = static_cast<TY*>(p.y) + m * p.ldy + n;
-          if (vec_ok && n + 4 <= p.N) {
-            *reinterpret_cast<Pack<TY, 4>*>(dst) = o;
-          } else {
-            for (int r = 0; r < 4; ++r)
-              if (n + r < p.N) dst[r] = o.v[r];
+      for (int i = i0; i < i0 + ni; ++i) {
+        const Pack<TY, OW> o = outputs(i, j, cj);
+        const int row = 16 * (wm * ni + i - i0) + (lane & 15);
+        const int col = kHalfCols ? col_of(j) / 2 : col_of(j);
+        *reinterpret_cast<Pack<TY, OW>*>(st + row * kStride + col * kOutBytes) = o;
+        if constexpr (EPI == kEpiSilu) {
+          if (p.absmax_parts != nullptr) {
+            // The row's 8 outputs of packed block nb lie in the four lanes
+            // l%16 + 16q.
+            float v = fmaxf(fabsf(to_f32(o.v[0])), fabsf(to_f32(o.v[1])));
+            v = fmaxf(v, __shfl_xor(v, 16));
+            v = fmaxf(v, __shfl_xor(v, 32));
+            const int64_t m = m0 + row_of(i);
+            const int64_t nb = static_cast<int64_t>(nb0) + wn * BC + j;
+            if (quad == 0 && m < p.M && nb < p.NB) p.absmax_parts[m * p.NB + nb] = v;
           }
         }
       }
     }
-  } else {
-    char* const st = static_cast<char*>(stage);
-    constexpr int EV = 16 / kOutBytes;    // outputs per 16-byte chunk
-    constexpr int CPR = kRowBytes / 16;   // chunks per tile row
-    constexpr int NT = WM * WN * 64;
-    constexpr int RPP = NT / CPR;         // rows per sweep; threads past RPP * CPR idle
-    static_assert(RPP >= 1, "a sweep covers at least one tile row");
-    const int64_t n_out_total = kHalfCols ? p.N / 2 : p.N;
-    const int64_t n0_out = kHalfCols ? n0 / 2 : n0;
-    const int crow = static_cast<int>(threadIdx.x) / CPR;
-    const int cchunk = static_cast<int>(threadIdx.x) % CPR;
-    const int64_t nc = n0_out + cchunk * EV;  // this thread's first output column
-    // Output row of tile-local row `row` of the pass over blocks i0 .. i0 + ni.
-    auto out_row = [&](int row, int i0, int ni) {
-      return m0 + 16 * (row / (16 * ni) * BR + i0) + row % (16 * ni);
-    };
-    // Residual add, y = dtype(dtype(dequant) + res); with ROOMY the pass's
-    // residual chunks (up to 8 per thread) are requested before its arithmetic.
-    // It spares O and down of a prefill layer a pass over their rows (three
-    // trips through memory).
-    constexpr bool kRes = EPI == kEpiDequant && kOutBytes == 2;
-    constexpr int kSweeps = (WM * 16 * IPP + RPP - 1) / RPP;
-    constexpr bool kEarly = kRes && ROOMY && kSweeps <= 8;
-    const bool res_vec = kRes && p.res != nullptr && nc + EV <= n_out_total &&
-                         ((reinterpret_cast<uintptr_t>(p.res) |
-                           static_cast<uintptr_t>(p.ld_res * kOutBytes)) & 15) == 0;
-    [[maybe_unused]] Pack<TY, EV> early[kEarly ? kSweeps : 1];
+    ring_barrier();
+    const int rows = WM * 16 * ni;
 #pragma unroll
-    for (int i0 = 0; i0 < BR; i0 += IPP) {
-      const int ni = BR - i0 < IPP ? BR - i0 : IPP;  // compile-time after unrolling
-      if constexpr (kEarly) {
-        if (res_vec) {
-#pragma unroll
-          for (int t = 0; t < kSweeps; ++t) {
-            const int row = t * RPP + crow;
-            const int64_t m = out_row(row, i0, ni);
-            const bool ok = crow < RPP && row < WM * 16 * ni && m < p.M;
-            early[t] = *reinterpret_cast<const Pack<TY, EV>*>(
-                static_cast<const TY*>(p.res) + (ok ? m : 0) * p.ld_res + nc);
-          }
-        }
-      }
-      ring_barrier();  // the ring's (or the last pass's) readers are done
-#pragma unroll
-      for (int j = 0; j < BC; ++j) {
-        const Cols cj = cols_of(j);
-#pragma unroll
-        for (int i = i0; i < i0 + ni; ++i) {
-          const Pack<TY, OW> o = outputs(i, j, cj);
-          const int row = 16 * (wm * ni + i - i0) + (lane & 15);
-          const int col = kHalfCols ? col_of(j) / 2 : col_of(j);
-          *reinterpret_cast<Pack<TY, OW>*>(st + row * kStride + col * kOutBytes) = o;
-          if constexpr (EPI == kEpiSilu) {
-            if (p.absmax_parts != nullptr) {
-              // The row's 8 outputs of packed block nb lie in the four lanes
-              // l%16 + 16q.
-              float v = fmaxf(fabsf(to_f32(o.v[0])), fabsf(to_f32(o.v[1])));
-              v = fmaxf(v, __shfl_xor(v, 16));
-              v = fmaxf(v, __shfl_xor(v, 32));
-              const int64_t m = m0 + row_of(i);
-              const int64_t nb = static_cast<int64_t>(nb0) + wn * BC + j;
-              if (quad == 0 && m < p.M && nb < p.NB) p.absmax_parts[m * p.NB + nb] = v;
-            }
-          }
-        }
-      }
-      ring_barrier();
-      const int rows = WM * 16 * ni;
-#pragma unroll
-      for (int base = 0; base < rows; base += RPP) {
-        const int row = base + crow;
-        const int64_t m = out_row(row, i0, ni);
-        const int64_t n = nc;
-        if (crow < RPP && row < rows && m < p.M && n < n_out_total) {
-          TY* const dst = static_cast<TY*>(p.y) + m * p.ldy + n;
-          Pack<TY, EV>& out = *reinterpret_cast<Pack<TY, EV>*>(st + row * kStride + cchunk * 16);
-          if constexpr (kRes) {
-            if (p.res != nullptr) {
-              const TY* const r = static_cast<const TY*>(p.res) + m * p.ld_res + n;
-              Pack<TY, EV> o = out;
-              if (res_vec) {
-                Pack<TY, EV> a;
-                if constexpr (kEarly) {
-                  a = early[base / RPP];
-                } else {
-                  a = *reinterpret_cast<const Pack<TY, EV>*>(r);
-                }
-#pragma unroll
-                for (int e = 0; e < EV; ++e) o.v[e] = add_rounded(o.v[e], a.v[e]);
+    for (int base = 0; base < rows; base += RPP) {
+      const int row = base + crow;
+      const int64_t m = out_row(row, i0, ni);
+      const int64_t n = nc;
+      if (crow < RPP && row < rows && m < p.M && n < n_out_total) {
+        TY* const dst = static_cast<TY*>(p.y) + m * p.ldy + n;
+        Pack<TY, EV>& out = *reinterpret_cast<Pack<TY, EV>*>(st + row * kStride + cchunk * 16);
+        if constexpr (kRes) {
+          if (p.res != nullptr) {
+            const TY* const r = static_cast<const TY*>(p.res) + m * p.ld_res + n;
+            Pack<TY, EV> o = out;
+            if (res_vec) {
+              Pack<TY, EV> a;
+              if constexpr (kEarly) {
+                a = early[base / RPP];
               } else {
-                for (int e = 0; e < EV; ++e)
-                  if (n + e < n_out_total) o.v[e] = add_rounded(o.v[e], r[e]);
+                a = *reinterpret_cast<const Pack<TY, EV>*>(r);
               }
-              out = o;
+#pragma unroll
+              for (int e = 0; e < EV; ++e) o.v[e] = add_rounded(o.v[e], a.v[e]);
+            } else {
+              for (int e = 0; e < EV; ++e)
+                if (n + e < n_out_total) o.v[e] = add_rounded(o.v[e], r[e]);
             }
+            out = o;
           }
-          const TY* const src = out.v;
-          if (vec_ok && n + EV <= n_out_total) {
-            *reinterpret_cast<i32x4*>(dst) = *reinterpret_cast<const i32x4*>(src);
-          } else {
-            for (int e = 0; e < EV; ++e)
-              if (n + e < n_out_total) dst[e] = src[e];
-          }
+        }
+        const TY* const src = out.v;
+        if (vec_ok && n + EV <= n_out_total) {
+          *reinterpret_cast<i32x4*>(dst) = *reinterpret_cast<const i32x4*>(src);
+        } else {
+          for (int e = 0; e < EV; ++e)
+            if (n + e < n_out_total) dst[e] = src[e];
         }
       }
     }
