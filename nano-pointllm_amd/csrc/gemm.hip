@@ -161,7 +161,9 @@ __global__ __launch_bounds__(WM * WN * 64, OCC * WM * WN / 4) void gemm_kernel(G
     wait_vmcnt<0>();
     ring_barrier();
   }
-  store_tile<WM, WN, BR, BC, kRing, EPI, TY, TH>(p, acc, wm, wn, mb0, nb0, lane, smem, scales);
+  constexpr bool kHoist = OCC * NW / 4 <= 4;  // at least 128 registers
+  store_tile<WM, WN, BR, BC, kRing, EPI, TY, TH, false, kHoist>(p, acc, wm, wn, mb0, nb0, lane, smem,
+                                                               scales);
 }
 
 // Weights-direct GEMM: NW wavefronts, each owning all A 16-row activation

@@ -149,7 +149,8 @@ __global__ __launch_bounds__(WM * WN * 64, WM * WN / 4) void gemm_pipe_kernel(Ge
   });
 
   wait_vmcnt<0>();  // copies past the last k-block, before the epilogue reuses the ring
-  store_tile<WM, WN, BR, BC, kRing, EPI, TY, TH, true>(p, acc, wm, wn, mb0, nb0, lane, smem, scales);
+  store_tile<WM, WN, BR, BC, kRing, EPI, TY, TH, true, false>(p, acc, wm, wn, mb0, nb0, lane, smem,
+                                                              scales);
 }
 
 // Launches a pipelined tile for the problem in p.

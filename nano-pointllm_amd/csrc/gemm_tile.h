@@ -142,8 +142,12 @@ struct TileScales {
 // from memory behind a bounds check, and 2-byte LDS writes) these took 32,
 // 16.6 and 47.  A 2048 x 22016 x 4096 SiLU product went from 191 to 177 us.
 // ROOMY: the kernel has registers for residual chunks beside its accumulators.
+// HOIST: and for the integer requant's twelve column operands of a block column,
+// read once for all its rows (1024 x 22016 x 768 40.5 us, 42.7 where they are read
+// for each block; on the 128 x 128 ring tile of 64 registers they spill, 2048 x
+// 4096 x 768 29 us against 21).
 template <int WM, int WN, int BR, int BC, int STAGE_BYTES, int EPI, typename TY, typename TH,
-          bool ROOMY = false>
+          bool ROOMY = false, bool HOIST = true>
 __device__ inline void store_tile(const GemmParams& p, i32x4 (&acc)[BR][BC], int wm, int wn,
                                   int mb0, int nb0, int lane, void* stage,
                                   const TileScales<EPI, 16 * WM * BR, 16 * WN * BC>& ts) {
@@ -176,12 +180,13 @@ __device__ inline void store_tile(const GemmParams& p, i32x4 (&acc)[BR][BC], int
   auto cols = [&](int k, int j) __attribute__((always_inline)) {
     return *reinterpret_cast<const Pack<float, 4>*>(&ts.col[k][col_of(j)]);
   };
+  constexpr bool kHoist = EPI != kEpiRequant || HOIST;
   struct Cols {
     Pack<float, 4> c[Scales::kCols > 0 ? Scales::kCols : 1];
   };
   auto cols_of = [&](int j) __attribute__((always_inline)) {
     Cols c;
-    if constexpr (Scales::kCols > 0 && EPI != kEpiRequant) {
+    if constexpr (Scales::kCols > 0 && kHoist) {
 #pragma unroll
       for (int k = 0; k < Scales::kCols; ++k) c.c[k] = cols(k, j);
     }
@@ -215,10 +220,12 @@ __device__ inline void store_tile(const GemmParams& p, i32x4 (&acc)[BR][BC], int
         } else if constexpr (EPI == kEpiDequant) {
           o.v[r] = from_f32<TY>(dequant1b(a[r], sx[i], cj.c[0].v[r], true, cj.c[1].v[r]));
         } else if constexpr (EPI == kEpiRequant) {
-          o.v[r] = static_cast<int8_t>(requant1(
-              a[r], __builtin_bit_cast(int32_t, ts.col[2][col_of(j) + r]),
-              __builtin_bit_cast(uint32_t, ts.col[0][col_of(j) + r]),
-              __builtin_bit_cast(int32_t, ts.col[1][col_of(j) + r])));
+          const auto col = [&](int k) {
+            return kHoist ? cj.c[k].v[r] : ts.col[k][col_of(j) + r];
+          };
+          o.v[r] = static_cast<int8_t>(
+              requant1(a[r], __builtin_bit_cast(int32_t, col(2)), __builtin_bit_cast(uint32_t, col(0)),
+                       __builtin_bit_cast(int32_t, col(1))));
         } else {
           static_assert(EPI == kEpiBf16Exact, "epilogue");
           o.v[r] = __builtin_bit_cast(
@@ -295,6 +302,7 @@ __device__ inline void store_tile(const GemmParams& p, i32x4 (&acc)[BR][BC], int
           }
         }
       }
+      if constexpr (EPI == kEpiRequant) __builtin_amdgcn_sched_barrier(0);
     }
     ring_barrier();
     const int rows = WM * 16 * ni;
