@@ -135,9 +135,9 @@ def test_other_weight_types_go_through_binary32(cuda):
 
 
 def test_rows_past_32_bit_columns(cuda):
-    """One row of 2^31 + 8 columns: every index past 32 bits, against the same
-    columns of a short row with the same scale, at both ends and around the
-    signed and unsigned 32-bit boundaries of bytes and elements."""
+    """One row of 2^31 + 8 columns against the same columns of a short row with
+    the same scale: the first ones, those around byte 2^31, and the last, past
+    element 2^31 and byte 2^32."""
     from nanopointllm_amd import w8a8
 
     k, n = (1 << 31) + 8, 4096
@@ -151,16 +151,16 @@ def test_rows_past_32_bit_columns(cuda):
             deq, s = w8a8.dynamic_per_token_activation_qdq(x)
         else:
             deq, q, s = w8a8.groupwise_weight_qdq(x, group_size=group)
-        for start in (0, (1 << 30) - n // 2, k - n - 8):
-            part = x[:, start:start + n].clone()
+        for start, end in ((0, n), ((1 << 30) - n // 2, (1 << 30) + n // 2), (k - n - 8, k)):
+            part = x[:, start:end].clone()
             if group is None:
                 part = torch.cat([part, x[:, 5:6]], dim=1)
                 want, ws = w8a8.dynamic_per_token_activation_qdq(part)
                 assert torch.equal(s, ws)
             else:
                 want, wq, ws = w8a8.groupwise_weight_qdq(part, group_size=group)
-                assert torch.equal(q[:, start:start + n], wq)
-                assert torch.equal(s[:, start // group:(start + n) // group], ws)
-            assert torch.equal(deq[:, start:start + n], want[:, :n])
+                assert torch.equal(q[:, start:end], wq)
+                assert torch.equal(s[:, start // group:-(-end // group)], ws)
+            assert torch.equal(deq[:, start:end], want[:, :end - start])
         del deq
     assert s.shape == (1, k // 128 + 1)
